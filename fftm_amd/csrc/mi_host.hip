@@ -1065,12 +1065,6 @@ struct fftm_mi_ffts_s
     }
 };
 
-namespace
-{
-constexpr int SHELL_BLOCKS = 512;
-constexpr int MAX_SHELLS   = 1024;
-} // namespace
-
 // Scratch of fftm_mi_ffts_shell_gradient_noalloc: the shell partial sums (SHELL_BLOCKS x
 // nshells doubles, 4 MiB at most), one copy per GPU for the life of the process.  Host
 // code never uses the array's name as an address: it uses the per-device pointer that
@@ -1126,36 +1120,78 @@ spec_geom make_spec_geom( const ffts_layout &L )
         kmax2 += ( L.n[a] / 2 ) * ( L.n[a] / 2 );
     }
     g.kmax2   = kmax2 > 0 ? kmax2 : 1; // all-ones sizes: every bin has k = 0
-    g.nshells = 1;
     if ( g.total < ( (int64_t)1 << 31 ) )
         for ( int m = 0; m < L.dim; ++m )
             div_magic( g.ext[m], g.mg[m], g.sh[m] );
     return g;
 }
 
-// grad[s] from the partial sums in `partials` (SHELL_BLOCKS x nshells doubles)
+// A walk over the bins with `threads` threads per block, at least four bins per thread where
+// there are enough, and at most max_blocks blocks (returned in `blocks`).
+spec_walk make_walk( const spec_geom &g, int threads, int64_t max_blocks, unsigned &blocks )
+{
+    spec_walk w{};
+    for ( int m = 0; m < 4; ++m )
+    {
+        const int k = m - ( 4 - g.nd ); // memory axis of the geometry
+        w.ext[m]    = k < 0 ? 1 : (int32_t)g.ext[k];
+        w.n[m]      = k < 0 || g.ax[k] == g.half_axis ? 0 : (int32_t)g.n[g.ax[k]];
+    }
+    w.dax   = -1;
+    w.total = g.total;
+    const int64_t nrows = g.total / w.ext[3];
+    // a block count that covers at least one row
+    int64_t nb = std::min<int64_t>( ( g.total + 4 * threads - 1 ) / ( 4 * threads ), max_blocks );
+    nb         = std::max<int64_t>( nb, ( w.ext[3] + threads - 1 ) / threads );
+    w.rows     = (int32_t)std::min<int64_t>( nb * threads / w.ext[3], nrows );
+    nb         = ( (int64_t)w.rows * w.ext[3] + threads - 1 ) / threads;
+    w.s2       = w.rows % w.ext[2];
+    w.s1       = w.rows / w.ext[2] % w.ext[1];
+    w.s0       = w.rows / w.ext[2] / w.ext[1];
+    blocks     = (unsigned)nb;
+    return w;
+}
+
+template <typename T>
+void launch_shell_gradient_t( fftm_mi_ffts_s *h, const void *grad_spectrum, const void *spectrum, void *grad,
+                              int nshells, double *partials )
+{
+    unsigned        blocks = 0;
+    const spec_walk w      = make_walk( h->sg, 512, SHELL_BLOCKS, blocks );
+    const size_t    lds    = sizeof( double ) * (size_t)nshells + sizeof( int ) * (size_t)( nshells + 1 );
+    hipLaunchKernelGGL( k_shell_partials<T>, dim3( blocks ), dim3( 512 ), lds, h->stream, w, nshells, h->sg.kmax2,
+                        static_cast<const cpx<T> *>( grad_spectrum ), static_cast<const cpx<T> *>( spectrum ), partials );
+    hipLaunchKernelGGL( k_shell_reduce<T>, dim3( ( nshells + 3 ) / 4 ), dim3( 256 ), 0, h->stream, partials,
+                        (int)blocks, nshells, static_cast<T *>( grad ) );
+}
+
+// grad[s] from the partial sums in `partials` (at most SHELL_BLOCKS x nshells doubles)
 void launch_shell_gradient( fftm_mi_ffts_s *h, const void *grad_spectrum, const void *spectrum, void *grad,
                             int nshells, double *partials )
 {
-    spec_geom g = h->sg;
-    g.nshells   = nshells;
-    const size_t lds = sizeof( double ) * (size_t)nshells;
     if ( h->prec == FFTM_MI_F32 )
-    {
-        hipLaunchKernelGGL( k_shell_partials<float>, dim3( SHELL_BLOCKS ), dim3( 256 ), lds, h->stream, g,
-                            static_cast<const cpx<float> *>( grad_spectrum ), static_cast<const cpx<float> *>( spectrum ),
-                            partials );
-        hipLaunchKernelGGL( k_shell_reduce<float>, dim3( ( nshells + 255 ) / 256 ), dim3( 256 ), 0, h->stream,
-                            partials, SHELL_BLOCKS, nshells, static_cast<float *>( grad ) );
-    }
+        launch_shell_gradient_t<float>( h, grad_spectrum, spectrum, grad, nshells, partials );
     else
+        launch_shell_gradient_t<double>( h, grad_spectrum, spectrum, grad, nshells, partials );
+}
+
+template <typename T>
+void launch_spectral_multiply( fftm_mi_ffts_s *h, const void *in, void *out, const void *filter, const void *coeffs,
+                               int nshells )
+{
+    const cpx<T> *src = static_cast<const cpx<T> *>( in );
+    cpx<T>       *dst = static_cast<cpx<T> *>( out );
+    if ( filter )
     {
-        hipLaunchKernelGGL( k_shell_partials<double>, dim3( SHELL_BLOCKS ), dim3( 256 ), lds, h->stream, g,
-                            static_cast<const cpx<double> *>( grad_spectrum ),
-                            static_cast<const cpx<double> *>( spectrum ), partials );
-        hipLaunchKernelGGL( k_shell_reduce<double>, dim3( ( nshells + 255 ) / 256 ), dim3( 256 ), 0, h->stream,
-                            partials, SHELL_BLOCKS, nshells, static_cast<double *>( grad ) );
+        const int64_t blocks = std::min<int64_t>( ( h->sg.total + 1023 ) / 1024, 8192 );
+        hipLaunchKernelGGL( k_filter_multiply<T>, dim3( (unsigned)blocks ), dim3( 256 ), 0, h->stream, h->sg.total, src,
+                            dst, static_cast<const T *>( filter ) );
+        return;
     }
+    unsigned        blocks = 0;
+    const spec_walk w      = make_walk( h->sg, 256, 4096, blocks );
+    hipLaunchKernelGGL( k_shell_multiply<T>, dim3( blocks ), dim3( 256 ), 0, h->stream, w, nshells, h->sg.kmax2, src,
+                        dst, static_cast<const T *>( coeffs ) );
 }
 } // namespace
 
@@ -1683,17 +1719,10 @@ int fftm_mi_ffts_spectral_multiply( fftm_mi_ffts h, const void *in, void *out, c
         return fail( FFTM_MI_INVALID_VALUE, "fftm_mi_ffts_spectral_multiply: pass exactly one of filter / shell_coeffs" );
     if ( shell_coeffs && ( nshells < 1 || nshells > MAX_SHELLS ) )
         return fail( FFTM_MI_INVALID_VALUE, "fftm_mi_ffts_spectral_multiply: nshells must be in 1..1024" );
-    spec_geom g = h->sg;
-    g.nshells   = shell_coeffs ? nshells : 1;
-    const int64_t blocks = std::min<int64_t>( ( g.total + 255 ) / 256, 8192 );
     if ( h->prec == FFTM_MI_F32 )
-        hipLaunchKernelGGL( k_spectral_multiply<float>, dim3( (unsigned)blocks ), dim3( 256 ), 0, h->stream, g,
-                            static_cast<const cpx<float> *>( in ), static_cast<cpx<float> *>( out ),
-                            static_cast<const float *>( filter ), static_cast<const float *>( shell_coeffs ) );
+        launch_spectral_multiply<float>( h, in, out, filter, shell_coeffs, nshells );
     else
-        hipLaunchKernelGGL( k_spectral_multiply<double>, dim3( (unsigned)blocks ), dim3( 256 ), 0, h->stream, g,
-                            static_cast<const cpx<double> *>( in ), static_cast<cpx<double> *>( out ),
-                            static_cast<const double *>( filter ), static_cast<const double *>( shell_coeffs ) );
+        launch_spectral_multiply<double>( h, in, out, filter, shell_coeffs, nshells );
     return spectral_launch_check( h, sync != 0, "fftm_mi_ffts_spectral_multiply" );
 }
 
@@ -1848,10 +1877,11 @@ int ensure_filter_chain( fftm_mi_ffts_s &h )
 template <typename T>
 int spectral_op_launch( fftm_mi_ffts_s &h, const filter_params<T> &f, const void *in, void *out )
 {
-    const int64_t total = h.sg.total;
-    const int64_t blocks = std::min<int64_t>( ( total + 255 ) / 256, 8192 );
-    hipLaunchKernelGGL( k_spectral_op<T>, dim3( (unsigned)std::max<int64_t>( blocks, 1 ) ), dim3( 256 ), 0, h.stream,
-                        f, static_cast<const cpx<T> *>( in ), static_cast<cpx<T> *>( out ), total );
+    unsigned  blocks = 0;
+    spec_walk w      = make_walk( h.sg, 256, 4096, blocks );
+    w.dax            = f.dax < 0 ? -1 : f.dax + ( 4 - h.sg.nd );
+    hipLaunchKernelGGL( k_spectral_op<T>, dim3( blocks ), dim3( 256 ), 0, h.stream, w, f,
+                        static_cast<const cpx<T> *>( in ), static_cast<cpx<T> *>( out ) );
     const hipError_t e = hipGetLastError();
     if ( e != hipSuccess )
         return fail( FFTM_MI_EXEC_FAILED, std::string( "fftm_mi: spectral operator launch failed: " ) + hipGetErrorString( e ) );
