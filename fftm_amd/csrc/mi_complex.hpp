@@ -197,82 +197,148 @@ __device__ __forceinline__ void dft3( cpx<T> *v )
     v[2]            = sub( t2, e );
 }
 
-template <bool INV, typename T>
-__device__ __forceinline__ void dft5( cpx<T> *v )
+// cos and sin of 2 pi m / R, m = 1 .. (R - 1) / 2
+template <int R>
+struct roots_of_unity;
+template <>
+struct roots_of_unity<5>
 {
-    const T c1 = (T)0.30901699437494742410229341718281906;  // cos(2pi/5)
-    const T c2 = (T)-0.80901699437494742410229341718281906; // cos(4pi/5)
-    const T s1 = (T)0.95105651629515357211643933337938214;  // sin(2pi/5)
-    const T s2 = (T)0.58778525229247312916870595463907277;  // sin(4pi/5)
-    const cpx<T> a1 = add( v[1], v[4] ), b1 = sub( v[1], v[4] );
-    const cpx<T> a2 = add( v[2], v[3] ), b2 = sub( v[2], v[3] );
-    const cpx<T> x0 = v[0];
-    const cpx<T> r1 = mk<T>( x0.x + c1 * a1.x + c2 * a2.x, x0.y + c1 * a1.y + c2 * a2.y );
-    const cpx<T> r2 = mk<T>( x0.x + c2 * a1.x + c1 * a2.x, x0.y + c2 * a1.y + c1 * a2.y );
-    // i_s * (s1 b1 + s2 b2), i_s * (s2 b1 - s1 b2)
-    const cpx<T> q1 = mul_si<INV>( mk<T>( s1 * b1.x + s2 * b2.x, s1 * b1.y + s2 * b2.y ) );
-    const cpx<T> q2 = mul_si<INV>( mk<T>( s2 * b1.x - s1 * b2.x, s2 * b1.y - s1 * b2.y ) );
-    v[0]            = mk<T>( x0.x + a1.x + a2.x, x0.y + a1.y + a2.y );
-    v[1]            = add( r1, q1 );
-    v[4]            = sub( r1, q1 );
-    v[2]            = add( r2, q2 );
-    v[3]            = sub( r2, q2 );
-}
+    static constexpr double c[] = { 0.309016994374947424102293417182819058, -0.80901699437494742410229341718281905 };
+    static constexpr double s[] = { 0.951056516295153572116439333379382143, 0.587785252292473129168705954639072768 };
+};
+template <>
+struct roots_of_unity<7>
+{
+    static constexpr double c[] = { 0.623489801858733530525004884004239810, -0.22252093395631440428890256449679475,
+                                    -0.90096886790241912623610231950744505 };
+    static constexpr double s[] = { 0.781831482468029808708444526674057750, 0.974927912181823607018131682993931217,
+                                    0.433883739117558120475768332848358754 };
+};
+template <>
+struct roots_of_unity<11>
+{
+    static constexpr double c[] = { 0.841253532831181168861811648919367717, 0.415415013001886425529274149229623203,
+                                    -0.14231483827328514044379266861636966, -0.65486073394528506405692507246629355,
+                                    -0.95949297361449738989036805706632769 };
+    static constexpr double s[] = { 0.540640817455597582107635954318691695, 0.909631995354518371411715383079028460,
+                                    0.989821441880932732376092037776718787, 0.755749574354258283774035843972344420,
+                                    0.281732556841429697711417915346616899 };
+};
+template <>
+struct roots_of_unity<13>
+{
+    static constexpr double c[] = { 0.885456025653209895900375522015098878, 0.568064746731155802511807559127516624,
+                                    0.120536680255323053349067687452543582, -0.35460488704253562596963789260001847,
+                                    -0.74851074817110109863463059970135138, -0.97094181742605202715698227629378922 };
+    static constexpr double s[] = { 0.464723172043768545656015335133104777, 0.822983865893656394579617423439381990,
+                                    0.992708874098053992800751649492520179, 0.935016242685414823439784599837830729,
+                                    0.663122658240795202376785492666766279, 0.239315664287557767148753726260211895 };
+};
 
-template <bool INV, typename T>
-__device__ __forceinline__ void dft7( cpx<T> *v )
+// Odd prime radix: the inputs q and R - q enter every output through their sum a_q and
+// difference b_q, y[m], y[R - m] = sum_q a_q cos(2 pi q m / R) +- s i sum_q b_q sin(...).
+template <int R, bool INV, typename T>
+__device__ __forceinline__ void dft_prime( cpx<T> *v )
 {
-    const T c1 = (T)0.62348980185873353052500488400423981;  // cos(2pi/7)
-    const T c2 = (T)-0.22252093395631440428890256449679476; // cos(4pi/7)
-    const T c3 = (T)-0.90096886790241912623610231950744505; // cos(6pi/7)
-    const T s1 = (T)0.78183148246802980870844452667405775;  // sin(2pi/7)
-    const T s2 = (T)0.97492791218182360701813168299393122;  // sin(4pi/7)
-    const T s3 = (T)0.43388373911755812047576833284835875;  // sin(6pi/7)
-    const cpx<T> a1 = add( v[1], v[6] ), b1 = sub( v[1], v[6] );
-    const cpx<T> a2 = add( v[2], v[5] ), b2 = sub( v[2], v[5] );
-    const cpx<T> a3 = add( v[3], v[4] ), b3 = sub( v[3], v[4] );
-    const cpx<T> x0 = v[0];
-    const cpx<T> r1 = mk<T>( x0.x + c1 * a1.x + c2 * a2.x + c3 * a3.x, x0.y + c1 * a1.y + c2 * a2.y + c3 * a3.y );
-    const cpx<T> r2 = mk<T>( x0.x + c2 * a1.x + c3 * a2.x + c1 * a3.x, x0.y + c2 * a1.y + c3 * a2.y + c1 * a3.y );
-    const cpx<T> r3 = mk<T>( x0.x + c3 * a1.x + c1 * a2.x + c2 * a3.x, x0.y + c3 * a1.y + c1 * a2.y + c2 * a3.y );
-    const cpx<T> q1 = mul_si<INV>(
-        mk<T>( s1 * b1.x + s2 * b2.x + s3 * b3.x, s1 * b1.y + s2 * b2.y + s3 * b3.y ) );
-    const cpx<T> q2 = mul_si<INV>(
-        mk<T>( s2 * b1.x - s3 * b2.x - s1 * b3.x, s2 * b1.y - s3 * b2.y - s1 * b3.y ) );
-    const cpx<T> q3 = mul_si<INV>(
-        mk<T>( s3 * b1.x - s1 * b2.x + s2 * b3.x, s3 * b1.y - s1 * b2.y + s2 * b3.y ) );
-    v[0] = mk<T>( x0.x + a1.x + a2.x + a3.x, x0.y + a1.y + a2.y + a3.y );
-    v[1] = add( r1, q1 );
-    v[6] = sub( r1, q1 );
-    v[2] = add( r2, q2 );
-    v[5] = sub( r2, q2 );
-    v[3] = add( r3, q3 );
-    v[4] = sub( r3, q3 );
-}
-
-// Generic radix R (any R <= 32): O(R^2) using the length-N twiddle table
-// (W_R^m = tw[m * N / R]).  Used for primes > 7 only.
-template <bool INV, typename T>
-__device__ __forceinline__ void dft_generic( cpx<T> *v, int R, const cpx<T> *__restrict__ tw, int64_t N )
-{
-    cpx<T>        o[32];
-    const int64_t step = N / R;
-    for ( int m = 0; m < R; ++m )
+    using W         = roots_of_unity<R>;
+    constexpr int H = ( R - 1 ) / 2;
+    cpx<T>        a[H], b[H];
+    const cpx<T>  x0 = v[0];
+    cpx<T>        y0 = x0;
+#pragma unroll
+    for ( int q = 0; q < H; ++q )
     {
-        cpx<T> s = mk<T>( 0, 0 );
-        for ( int q = 0; q < R; ++q )
-        {
-            const cpx<T> w = tw[( ( q * m ) % R ) * step];
-            s              = add( s, twmul<INV>( v[q], w ) );
-        }
-        o[m] = s;
+        a[q] = add( v[q + 1], v[R - 1 - q] );
+        b[q] = sub( v[q + 1], v[R - 1 - q] );
+        y0   = add( y0, a[q] );
     }
-    for ( int m = 0; m < R; ++m )
-        v[m] = o[m];
+    v[0] = y0;
+#pragma unroll
+    for ( int m = 1; m <= H; ++m )
+    {
+        cpx<T> r = x0, t = mk<T>( 0, 0 );
+#pragma unroll
+        for ( int q = 1; q <= H; ++q )
+        {
+            const int e = q * m % R;
+            const T   c = (T)W::c[( e <= H ? e : R - e ) - 1];
+            const T   s = e <= H ? (T)W::s[e - 1] : -(T)W::s[R - e - 1];
+            r           = mk<T>( fmat( c, a[q - 1].x, r.x ), fmat( c, a[q - 1].y, r.y ) );
+            t           = q == 1 ? scl( b[0], s ) : mk<T>( fmat( s, b[q - 1].x, t.x ), fmat( s, b[q - 1].y, t.y ) );
+        }
+        t        = mul_si<INV>( t );
+        v[m]     = add( r, t );
+        v[R - m] = sub( r, t );
+    }
 }
 
 template <int R, bool INV, typename T>
-__device__ __forceinline__ void dft_fixed( cpx<T> *v, const cpx<T> *__restrict__ tw, int64_t N )
+__device__ __forceinline__ void dft_fixed( cpx<T> *v );
+
+// R = A B with coprime factors (Good 1958, Thomas 1963): input n = n1 B + n2 A mod R and
+// output k = k1 mod A = k2 mod B turn the DFT into A x B with no twiddles.
+template <int A, int B, bool INV, typename T>
+__device__ __forceinline__ void dft_coprime( cpx<T> *v )
+{
+    constexpr int R = A * B;
+    cpx<T>        y[A][B];
+#pragma unroll
+    for ( int n2 = 0; n2 < B; ++n2 )
+    {
+        cpx<T> u[A];
+#pragma unroll
+        for ( int n1 = 0; n1 < A; ++n1 )
+            u[n1] = v[( n1 * B + n2 * A ) % R];
+        dft_fixed<A, INV>( u );
+#pragma unroll
+        for ( int k1 = 0; k1 < A; ++k1 )
+            y[k1][n2] = u[k1];
+    }
+#pragma unroll
+    for ( int k1 = 0; k1 < A; ++k1 )
+    {
+        dft_fixed<B, INV>( y[k1] );
+#pragma unroll
+        for ( int k = 0; k < R; ++k )
+            if ( k % A == k1 )
+                v[k] = y[k1][k % B];
+    }
+}
+
+// radix 9 = 3 x 3 with the twiddles W9, W9^2, W9^4
+template <bool INV, typename T>
+__device__ __forceinline__ void dft9( cpx<T> *v )
+{
+    const T      sg = INV ? (T)1 : (T)-1;
+    const cpx<T> w1 = mk<T>( (T)0.766044443118978035202392650555416673, sg * (T)0.642787609686539326322643409907263432 );
+    const cpx<T> w2 = mk<T>( (T)0.173648177666930348851716626769314796, sg * (T)0.984807753012208059366743024589523013 );
+    const cpx<T> w4 = mk<T>( (T)-0.93969262078590838405410927732473146, sg * (T)0.342020143325668733044099614682259580 );
+    cpx<T>       y[3][3];
+#pragma unroll
+    for ( int n2 = 0; n2 < 3; ++n2 )
+    {
+        cpx<T> u[3] = { v[n2], v[n2 + 3], v[n2 + 6] };
+        dft3<INV>( u );
+#pragma unroll
+        for ( int k1 = 0; k1 < 3; ++k1 )
+            y[k1][n2] = u[k1];
+    }
+    y[1][1] = mul( y[1][1], w1 );
+    y[1][2] = mul( y[1][2], w2 );
+    y[2][1] = mul( y[2][1], w2 );
+    y[2][2] = mul( y[2][2], w4 );
+#pragma unroll
+    for ( int k1 = 0; k1 < 3; ++k1 )
+    {
+        dft3<INV>( y[k1] );
+#pragma unroll
+        for ( int k2 = 0; k2 < 3; ++k2 )
+            v[k1 + 3 * k2] = y[k1][k2];
+    }
+}
+
+template <int R, bool INV, typename T>
+__device__ __forceinline__ void dft_fixed( cpx<T> *v )
 {
     if constexpr ( R == 2 )
         dft2<INV>( v );
@@ -280,33 +346,26 @@ __device__ __forceinline__ void dft_fixed( cpx<T> *v, const cpx<T> *__restrict__
         dft3<INV>( v );
     else if constexpr ( R == 4 )
         dft4<INV>( v );
-    else if constexpr ( R == 5 )
-        dft5<INV>( v );
-    else if constexpr ( R == 7 )
-        dft7<INV>( v );
+    else if constexpr ( R == 5 || R == 7 || R == 11 || R == 13 )
+        dft_prime<R, INV>( v );
+    else if constexpr ( R == 6 )
+        dft_coprime<2, 3, INV>( v );
     else if constexpr ( R == 8 )
         dft8<INV>( v );
+    else if constexpr ( R == 9 )
+        dft9<INV>( v );
+    else if constexpr ( R == 10 )
+        dft_coprime<2, 5, INV>( v );
+    else if constexpr ( R == 12 )
+        dft_coprime<4, 3, INV>( v );
+    else if constexpr ( R == 14 )
+        dft_coprime<2, 7, INV>( v );
+    else if constexpr ( R == 15 )
+        dft_coprime<3, 5, INV>( v );
     else if constexpr ( R == 16 )
         dft16<INV>( v );
     else
-        dft_generic<INV>( v, R, tw, N );
-}
-
-// Runtime-radix dispatch (generic kernel)
-template <bool INV, typename T>
-__device__ __forceinline__ void dft_runtime( cpx<T> *v, int R, const cpx<T> *__restrict__ tw, int64_t N )
-{
-    switch ( R )
-    {
-    case 2: dft2<INV>( v ); break;
-    case 3: dft3<INV>( v ); break;
-    case 4: dft4<INV>( v ); break;
-    case 5: dft5<INV>( v ); break;
-    case 7: dft7<INV>( v ); break;
-    case 8: dft8<INV>( v ); break;
-    case 16: dft16<INV>( v ); break;
-    default: dft_generic<INV>( v, R, tw, N ); break;
-    }
+        static_assert( R == 1, "no butterfly of this radix" );
 }
 
 // ---------------------------------------------------------------------------

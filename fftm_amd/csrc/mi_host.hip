@@ -69,8 +69,7 @@ struct pass_rt
     int64_t    d0 = 1, d1 = 1, is0 = 0, is1 = 0, is2 = 0, os0 = 0, os1 = 0, os2 = 0;
     bool       loadb  = false, storeb = false;
     bool       generic = false;
-    radix_list rl{};
-    int        gen_cols = 1;
+    any_plan   any{};   // generic: the length's runtime schedule and tile
     int        wmode    = 0; // real-axis bin weights (adjoints), see pass_params::wmode
     int        var      = 0; // tile-shape variant of the fixed-length kernel
     bool       rev      = false; // tiles in reverse order (alternate passes of a transform pair)
@@ -95,43 +94,110 @@ bool is_pow2( int64_t n )
     return n >= 1 && ( n & ( n - 1 ) ) == 0;
 }
 
-// radices for the generic kernel (each <= 16); false if N has a prime factor > 13
-bool generic_radices( int64_t N, radix_list &rl )
-{
-    rl.n      = 0;
-    int64_t m = N;
-    int     k = 0;
-    while ( m % 2 == 0 )
-    {
-        m /= 2;
-        ++k;
-    }
-    while ( k >= 4 )
-    {
-        rl.r[rl.n++] = 16;
-        k -= 4;
-    }
-    if ( k == 3 )
-        rl.r[rl.n++] = 8;
-    else if ( k == 2 )
-        rl.r[rl.n++] = 4;
-    else if ( k == 1 )
-        rl.r[rl.n++] = 2;
-    const int primes[] = { 3, 5, 7, 11, 13 };
-    for ( int p : primes )
-        while ( m % p == 0 )
-        {
-            if ( rl.n >= 20 )
-                return false;
-            rl.r[rl.n++] = p;
-            m /= p;
-        }
-    return m == 1;
-}
-
 int csize_of( int prec )
 {
     return prec == FFTM_MI_F32 ? 8 : 16;
+}
+
+// The schedule of a runtime-length pass: as few of the kernel's radices as multiply to N.
+// Among those, the first one first by the LDS bank conflicts of stage 0's writes, which have
+// its stride (an odd radix none, twice an odd one two-fold), then the most even ones (the
+// smallest sum).  best.n = 0 if there is none.
+struct any_schedule
+{
+    int n = 0, cost = 0, r[ANY_MAX_STAGES] = {};
+};
+
+void any_radices( int64_t N, int csize, int maxr, any_schedule cur, any_schedule &best )
+{
+    if ( N == 1 )
+    {
+        int first = 0;
+        for ( int i = 1; i < cur.n; ++i )
+            if ( ( cur.r[i] & -cur.r[i] ) < ( cur.r[first] & -cur.r[first] ) )
+                first = i;
+        const int conflict = cur.r[first] & -cur.r[first];
+        std::swap( cur.r[0], cur.r[first] );
+        cur.cost = ( conflict > 2 ? conflict * 100 : 0 );
+        for ( int i = 0; i < cur.n; ++i )
+            cur.cost += cur.r[i];
+        if ( best.n == 0 || cur.n < best.n || ( cur.n == best.n && cur.cost < best.cost ) )
+            best = cur;
+        return;
+    }
+    if ( cur.n == ANY_MAX_STAGES || ( best.n && cur.n == best.n ) )
+        return;
+    for ( int r = maxr; r >= 2; --r )
+        if ( N % r == 0 && any_radix( r, csize ) )
+        {
+            any_schedule next = cur;
+            next.r[next.n++]  = r;
+            any_radices( N / r, csize, r, next, best );
+        }
+}
+
+uint32_t mulhi_magic( int64_t d )
+{
+    return d > 1 ? (uint32_t)( ( ( (uint64_t)1 << 32 ) / (uint64_t)d ) + 1 ) : 0;
+}
+
+// Schedule and tile of a runtime-length pass; false if the length is out of range.
+bool make_any_plan( int64_t N, int csize, bool loadb, int kind, any_plan &a )
+{
+    a    = any_plan{};
+    a.N  = (int32_t)N;
+    a.nh = (int32_t)( N / 2 + 1 );
+    any_schedule sch;
+    if ( N == 1 )
+        sch.r[sch.n++] = 1;
+    else
+        any_radices( N, csize, 16, any_schedule{}, sch );
+    if ( sch.n == 0 )
+        return false;
+    int per = any_values( csize ) + 3; // values per thread that whole butterflies of every stage allow
+    a.nst   = sch.n;
+    int64_t ns = 1;
+    for ( int i = 0; i < sch.n; ++i )
+    {
+        const int r   = sch.r[i];
+        per           = std::min( per, any_butterflies( r, csize ) * r );
+        a.s[i].r      = r;
+        a.s[i].ns     = (int32_t)ns;
+        a.s[i].nbf    = (int32_t)( N / r );
+        a.s[i].tst    = (int32_t)( N / ( ns * r ) );
+        a.s[i].mg_nbf = mulhi_magic( N / r );
+        a.s[i].mg_ns  = mulhi_magic( ns );
+        if ( r > 1 && !any_common_radix( r, csize ) )
+            a.rare = 1;
+        ns *= r;
+    }
+    a.mg_n  = mulhi_magic( N );
+    a.mg_nh = mulhi_magic( a.nh );
+    const int64_t line = std::max<int64_t>( N, kind == KIND_C2R ? 2 * a.nh : 0 ); // LDS values per line (pair)
+    int           cols;
+    if ( loadb )
+    {
+        // one 128-byte row segment, narrower where the tile would not fit 64 KB, wider for
+        // short lines
+        cols = 128 / csize;
+        while ( cols > 1 && ( line * cols * csize > 65536 || N * cols > (int64_t)per * any_max_threads( csize ) ) )
+            cols /= 2;
+        while ( cols < 64 && N * cols / per < 256 && N * cols * csize <= 16384 )
+            cols *= 2;
+        while ( ( 1 << a.csh ) < cols )
+            ++a.csh;
+    }
+    else
+    {
+        cols = (int)std::max<int64_t>( 1, 256 * per / N );
+        while ( cols > 1 && line * cols * csize > 32768 )
+            --cols;
+    }
+    a.cols    = cols;
+    a.mg_cols = mulhi_magic( cols );
+    a.elems   = (int32_t)( line * cols );
+    a.nt      = (int32_t)( ( ( N * cols + per - 1 ) / per + 63 ) / 64 * 64 );
+    return a.nt <= any_max_threads( csize );
 }
 
 // Decide how a pass of length N runs (fixed kernel or generic); fills N-dependent fields.
@@ -142,19 +208,19 @@ int configure_kernel( pass_rt &p, int prec )
         p.generic = false;
         return ok();
     }
-    if ( !generic_radices( p.N, p.rl ) )
+    int64_t m = p.N;
+    for ( int f : { 2, 3, 5, 7, 11, 13 } )
+        while ( m % f == 0 )
+            m /= f;
+    if ( m != 1 )
         return fail( FFTM_MI_NOT_SUPPORTED,
                      "fftm_mi: transform length " + std::to_string( p.N ) +
                          " has a prime factor above 13 (not supported yet)" );
-    const int cs   = csize_of( prec );
-    int       cols = prec == FFTM_MI_F32 ? 16 : 8;
-    while ( cols > 1 && 2 * p.N * cols * cs > 65536 )
-        cols /= 2;
-    if ( 2 * p.N * cols * cs > 65536 )
+    const int cs = csize_of( prec );
+    if ( 2 * p.N * cs > 65536 || !make_any_plan( p.N, cs, p.loadb, p.kind, p.any ) )
         return fail( FFTM_MI_NOT_SUPPORTED,
                      "fftm_mi: transform length " + std::to_string( p.N ) + " exceeds the single-pass limit" );
-    p.generic  = true;
-    p.gen_cols = cols;
+    p.generic = true;
     return ok();
 }
 
@@ -392,14 +458,14 @@ hipError_t launch_one( const pass_rt &r, const tables &tb, const void *src, void
             return launch_pass_rs_f32( p, (int)r.N, r.inv, shape, rs, IO_F32, s );
         if ( r.filter )
             return launch_filter_f32( p, *static_cast<const filter_params<float> *>( filter ), (int)r.N, r.loadb, shape, s );
-        return r.generic ? launch_generic_f32( p, r.rl, (int)r.N, r.gen_cols, r.kind, r.inv, s )
+        return r.generic ? launch_any_f32( p, r.any, r.kind, r.inv, r.loadb, s )
                          : launch_pass_f32( p, (int)r.N, r.kind, r.inv, r.loadb, shape, s );
     }
     else
     {
         if ( r.filter )
             return launch_filter_f64( p, *static_cast<const filter_params<double> *>( filter ), (int)r.N, r.loadb, shape, s );
-        return r.generic ? launch_generic_f64( p, r.rl, (int)r.N, r.gen_cols, r.kind, r.inv, s )
+        return r.generic ? launch_any_f64( p, r.any, r.kind, r.inv, r.loadb, s )
                          : launch_pass_f64( p, (int)r.N, r.kind, r.inv, r.loadb, shape, s );
     }
 }

@@ -1,5 +1,5 @@
 // Dispatch of the fixed-length pass kernels (one definition per length lives in the
-// mi_kernels_<prec>_<group>.hip units) and the generic kernel launchers.
+// mi_kernels_<prec>_<group>.hip units).
 #include "mi_kernels_impl.hpp"
 
 #define FFTM_MI_LENGTHS( X, T, TN )                                                                                    \
@@ -165,18 +165,6 @@ hipError_t launch_pass_rs_f32( const pass_params<float> &p, int N, bool inv, int
     case 1024: return launch_rs_f32_n1024( p, inv, shape, rs, iom, s );
     default: return hipErrorInvalidValue;
     }
-}
-
-hipError_t launch_generic_f32( const pass_params<float> &p, const radix_list &rl, int N, int cols, int kind, bool inv,
-                               hipStream_t s )
-{
-    return detail::launch_generic_t<float>( p, rl, N, cols, kind, inv, s );
-}
-
-hipError_t launch_generic_f64( const pass_params<double> &p, const radix_list &rl, int N, int cols, int kind, bool inv,
-                               hipStream_t s )
-{
-    return detail::launch_generic_t<double>( p, rl, N, cols, kind, inv, s );
 }
 
 } // namespace fftm_mi

@@ -205,33 +205,6 @@ hipError_t launch_mixed_n( const pass_params<float> &p, int kind, bool inv, bool
     }
 }
 
-template <typename T>
-hipError_t launch_generic_t( const pass_params<T> &p, const radix_list &rl, int N, int cols, int kind, bool inv,
-                             hipStream_t s )
-{
-    const int64_t cpt    = kind == KIND_C2C ? 1 : 2;
-    const int64_t per    = (int64_t)cols * cpt;
-    const int64_t ntiles = ( p.ncols + per - 1 ) / per;
-    if ( ntiles <= 0 )
-        return hipSuccess;
-    if ( ntiles > 0x7fffffffLL )
-        return hipErrorInvalidConfiguration;
-    const size_t lds = 2 * (size_t)N * (size_t)cols * sizeof( cpx<T> );
-    const dim3   grid( (unsigned)ntiles ), block( GEN_THREADS );
-    if ( kind == KIND_C2C )
-    {
-        if ( inv )
-            hipLaunchKernelGGL( ( k_pass_generic<T, KIND_C2C, true> ), grid, block, lds, s, p, rl, N, cols );
-        else
-            hipLaunchKernelGGL( ( k_pass_generic<T, KIND_C2C, false> ), grid, block, lds, s, p, rl, N, cols );
-    }
-    else if ( kind == KIND_R2C )
-        hipLaunchKernelGGL( ( k_pass_generic<T, KIND_R2C, false> ), grid, block, lds, s, p, rl, N, cols );
-    else
-        hipLaunchKernelGGL( ( k_pass_generic<T, KIND_C2R, true> ), grid, block, lds, s, p, rl, N, cols );
-    return hipGetLastError();
-}
-
 // Alternative radix schedules (RS 1: make_rplan_alt on the vector ALUs, RS 2: its radix-16
 // stage on the matrix cores) of the strided C2C passes, FP32 arithmetic with FP32 or
 // FP16-stored lines, tile shapes 0 and 6 (schedule 1 also in shape 2).

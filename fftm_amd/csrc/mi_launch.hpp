@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "mi_any.hpp"
 #include "mi_pass.hpp"
 #include "mi_plane.hpp"
 
@@ -85,9 +86,8 @@ hipError_t launch_filter_f32( const pass_params<float> &p, const filter_params<f
 hipError_t launch_filter_f64( const pass_params<double> &p, const filter_params<double> &f, int N, bool loadb, int var,
                               hipStream_t s );
 
-hipError_t launch_generic_f32( const pass_params<float> &p, const radix_list &rl, int N, int cols, int kind, bool inv,
-                               hipStream_t s );
-hipError_t launch_generic_f64( const pass_params<double> &p, const radix_list &rl, int N, int cols, int kind, bool inv,
-                               hipStream_t s );
+// lengths without a compiled kernel (mi_any.hpp)
+hipError_t launch_any_f32( const pass_params<float> &p, const any_plan &a, int kind, bool inv, bool loadb, hipStream_t s );
+hipError_t launch_any_f64( const pass_params<double> &p, const any_plan &a, int kind, bool inv, bool loadb, hipStream_t s );
 
 } // namespace fftm_mi

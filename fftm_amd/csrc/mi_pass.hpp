@@ -236,13 +236,6 @@ struct pass_ctx
     bool                    va, vb;
 };
 
-// Runtime description for the generic (any-radix) kernel.
-struct radix_list
-{
-    int32_t n;      // number of stages
-    int32_t r[20];  // radices (<= 16 each)
-};
-
 // ---------------------------------------------------------------------------
 // compile-time radix schedule for a given N
 // ---------------------------------------------------------------------------
@@ -1251,7 +1244,7 @@ struct pass_kernel
                     if constexpr ( MF )
                         dft16_mfma( reinterpret_cast<cpx<float>( & )[16]>( w[b] ), am );
                     else
-                        dft_fixed<R2, INV>( w[b], x.p->tw, N );
+                        dft_fixed<R2, INV>( w[b] );
                 }
             }
             __syncthreads();
@@ -1273,7 +1266,7 @@ struct pass_kernel
         {
             const int j = jmap<0>( x.t, b );
             if ( NBF0 % TPC == 0 || j < NBF0 )
-                dft_fixed<R0, INV>( v[b], x.p->tw, N );
+                dft_fixed<R0, INV>( v[b] );
         }
         __syncthreads();
         chain<0, NB0, R0>( v, x );
@@ -1462,7 +1455,7 @@ struct pass_kernel
                         }
                         v[b][r] = mk<T>( a.x - bq.y, a.y + bq.x );
                     }
-                    dft_fixed<R0, INV>( v[b], p.tw, N );
+                    dft_fixed<R0, INV>( v[b] );
                 }
             }
             __syncthreads(); // the exchange buffer aliases the staging area
@@ -1502,8 +1495,8 @@ struct pass_kernel
                                 v[b + 1][r]     = mk<T>( q.z, q.w );
                             }
                         }
-                        dft_fixed<R0, INV>( v[b], p.tw, N );
-                        dft_fixed<R0, INV>( v[b + 1], p.tw, N );
+                        dft_fixed<R0, INV>( v[b] );
+                        dft_fixed<R0, INV>( v[b + 1] );
                     }
                 }
                 loaded = true;
@@ -1579,7 +1572,7 @@ struct pass_kernel
                                 h = __builtin_bit_cast( HE, v[b][r].x );
                             v[b][r] = x.va ? h16_decode<SPL>( h, e ) : mk<float>( 0, 0 );
                         }
-                        dft_fixed<R0, INV>( v[b], p.tw, N );
+                        dft_fixed<R0, INV>( v[b] );
                     }
                 }
                 loaded = true;
@@ -1677,7 +1670,7 @@ struct pass_kernel
                                 h = __builtin_bit_cast( HE, v[b][r].x );
                             v[b][r] = h16_decode<SPL>( h, e );
                         }
-                        dft_fixed<R0, INV>( v[b], p.tw, N );
+                        dft_fixed<R0, INV>( v[b] );
                     }
                 }
                 loaded = true;
@@ -1699,7 +1692,7 @@ struct pass_kernel
                         else
                             v[b][r] = load_line<KIND>( p, x.ia, x.ib, x.va, x.vb, j + r * NBF0, N );
                     }
-                    dft_fixed<R0, INV>( v[b], p.tw, N );
+                    dft_fixed<R0, INV>( v[b] );
                 }
             }
         }
@@ -1721,111 +1714,6 @@ __global__ void __launch_bounds__( ( pass_kernel<T, N, KIND_C2C, false, LOADB, V
     k_pass_filter( const pass_params<T> p, const filter_params<T> f )
 {
     pass_kernel<T, N, KIND_C2C, false, LOADB, VAR, IO_F32, true>::run( p, &f );
-}
-
-// ---------------------------------------------------------------------------
-// Generic kernel: runtime N and radix list (radices <= 16), ping-pong LDS,
-// column-fastest mapping.  Used for lengths without a compiled specialisation.
-// ---------------------------------------------------------------------------
-constexpr int GEN_THREADS = 256;
-
-template <typename T, int R, bool INV>
-__device__ __forceinline__ void gen_stage( const cpx<T> *src, cpx<T> *dst, int N, int Ns, int tw_cols, int c,
-                                           int t, int tpc, const cpx<T> *__restrict__ tw )
-{
-    const int nbf = N / R;
-    for ( int j = t; j < nbf; j += tpc )
-    {
-        cpx<T> v[R];
-        for ( int r = 0; r < R; ++r )
-            v[r] = src[( j + r * nbf ) * tw_cols + c];
-        const int k    = j % Ns;
-        const int tstp = N / ( Ns * R );
-        for ( int r = 1; r < R; ++r )
-            v[r] = twmul<INV>( v[r], tw[r * k * tstp] );
-        dft_fixed<R, INV>( v, tw, N );
-        const int d = ( j / Ns ) * Ns * R + k;
-        for ( int m = 0; m < R; ++m )
-            dst[( d + m * Ns ) * tw_cols + c] = v[m];
-    }
-}
-
-template <typename T, bool INV>
-__device__ __forceinline__ void gen_stage_rt( int R, const cpx<T> *src, cpx<T> *dst, int N, int Ns, int tw_cols,
-                                              int c, int t, int tpc, const cpx<T> *__restrict__ tw )
-{
-    switch ( R )
-    {
-    case 2: gen_stage<T, 2, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    case 3: gen_stage<T, 3, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    case 4: gen_stage<T, 4, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    case 5: gen_stage<T, 5, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    case 7: gen_stage<T, 7, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    case 8: gen_stage<T, 8, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    case 11: gen_stage<T, 11, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    case 13: gen_stage<T, 13, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    case 16: gen_stage<T, 16, INV>( src, dst, N, Ns, tw_cols, c, t, tpc, tw ); break;
-    default: break; // host never plans other radices
-    }
-}
-
-template <typename T, int KIND, bool INV>
-__global__ void __launch_bounds__( GEN_THREADS )
-    k_pass_generic( const pass_params<T> p, const radix_list rl, int N, int tw_cols )
-{
-    extern __shared__ unsigned char gen_lds_raw[];
-    cpx<T>       *buf0 = reinterpret_cast<cpx<T> *>( gen_lds_raw );
-    cpx<T>       *buf1 = buf0 + (int64_t)N * tw_cols;
-    constexpr int CPT  = KIND == KIND_C2C ? 1 : 2;
-    const int     tid  = threadIdx.x;
-    const int     tpc  = GEN_THREADS / tw_cols;
-    const int     c    = tid % tw_cols;
-    const int     t    = tid / tw_cols;
-    const int64_t tile = xcd_tile( blockIdx.x, gridDim.x );
-    const int64_t col  = ( tile * tw_cols + c ) * CPT;
-    const bool    va   = c < tw_cols && col < p.ncols;
-    const bool    vb   = CPT == 2 && c < tw_cols && col + 1 < p.ncols;
-    int64_t       ia = 0, oa = 0, ib = 0, ob = 0;
-    col_offsets( p, col, ia, oa );
-    if ( CPT == 2 )
-        col_offsets( p, col + 1, ib, ob );
-    if ( t < tpc )
-        for ( int n = t; n < N; n += tpc )
-            buf0[n * tw_cols + c] = load_line<KIND>( p, ia, ib, va, vb, n, N );
-    __syncthreads();
-    cpx<T> *src = buf0, *dst = buf1;
-    int     Ns  = 1;
-    for ( int s = 0; s < rl.n; ++s )
-    {
-        if ( t < tpc )
-            gen_stage_rt<T, INV>( rl.r[s], src, dst, N, Ns, tw_cols, c, t, tpc, p.tw );
-        __syncthreads();
-        Ns *= rl.r[s];
-        cpx<T> *tmp = src;
-        src         = dst;
-        dst         = tmp;
-    }
-    if ( t >= tpc )
-        return;
-    if constexpr ( KIND == KIND_R2C )
-    {
-        cpx<T> *out = static_cast<cpx<T> *>( p.out );
-        for ( int k = t; k <= N / 2; k += tpc )
-        {
-            const T      h  = ( p.wmode == 1 && k != 0 && 2 * k != N ) ? p.scale : (T)0.5 * p.scale;
-            const cpx<T> zk = src[k * tw_cols + c];
-            const cpx<T> zm = src[( k == 0 ? 0 : N - k ) * tw_cols + c];
-            if ( va )
-                out[oa + (int64_t)k * p.oes] = mk<T>( h * ( zk.x + zm.x ), h * ( zk.y - zm.y ) );
-            if ( vb )
-                out[ob + (int64_t)k * p.oes] = mk<T>( h * ( zk.y + zm.y ), h * ( zm.x - zk.x ) );
-        }
-    }
-    else
-    {
-        for ( int n = t; n < N; n += tpc )
-            store_line<KIND>( p, oa, ob, va, vb, n, src[n * tw_cols + c] );
-    }
 }
 
 } // namespace fftm_mi

@@ -102,7 +102,7 @@ __device__ __forceinline__ void lds_lines( cpx<T> *buf, int es, int ls, int gs, 
                     for ( int r = 1; r < R; ++r )
                         v[i][r] = twmul<INV>( v[i][r], tw[r * k * TST] );
                 }
-                dft_fixed<R, INV>( v[i], tw, N );
+                dft_fixed<R, INV>( v[i] );
             }
         }
         __syncthreads();
@@ -437,7 +437,7 @@ struct rx_lines
                     for ( int r = 1; r < R; ++r )
                         v[i][r] = twmul<INV>( v[i][r], tw[r * k * TST] );
                 }
-                dft_fixed<R, INV>( v[i], tw, N );
+                dft_fixed<R, INV>( v[i] );
             }
         }
         if constexpr ( S == 0 )
