@@ -425,8 +425,9 @@ constexpr geom pick_geom( int N, int csize, bool loadb, int var = 0 )
         if ( tpc < lo )
             tpc = lo;
         // two butterflies per thread when the tile still fits: the first and last stages
-        // then move pairs of consecutive elements (8- or 16-byte accesses)
-        if ( tpc >= 2 && tpc / 2 >= lo && ( 256 / ( tpc / 2 ) ) * geom_pa( N, 3 ) * csize <= lds_limit_bytes() )
+        // then move pairs of consecutive elements (8- or 16-byte accesses).  Not with FP64
+        // radix 16: 32 values are 128 registers
+        if ( ( csize == 8 || rm <= 8 ) && tpc >= 2 && tpc / 2 >= lo && ( 256 / ( tpc / 2 ) ) * geom_pa( N, 3 ) * csize <= lds_limit_bytes() )
             tpc /= 2;
         int tw  = 256 / tpc > 0 ? 256 / tpc : 1;
         int pad = 3;
@@ -642,6 +643,27 @@ __device__ __forceinline__ void store_line( const pass_params<T> &p, int64_t oa,
         if ( vb )
             dst[ob + (int64_t)n * p.oes] = z.y * p.scale;
     }
+}
+
+// Copy n16 16-byte pieces from HBM straight into LDS (both 16-byte aligned), nt threads
+// together: piece e goes from src + 16 e to dst + 16 e.  The loads write LDS without passing
+// through registers, so a thread can have all of its pieces in flight at once.  The caller's
+// next barrier must be stage_wait's.
+__device__ __forceinline__ void stage_copy16( const void *src, void *dst, int n16, int tid, int nt )
+{
+    typedef __attribute__( ( address_space( 1 ) ) ) const uint32_t *gptr;
+    typedef __attribute__( ( address_space( 3 ) ) ) uint32_t       *lptr;
+    // the LDS address of a wave's load is that of its first lane, the lanes follow
+    const int first = __builtin_amdgcn_readfirstlane( tid );
+    for ( int e = 0; e + first < n16; e += nt )
+        if ( e + tid < n16 )
+            __builtin_amdgcn_global_load_lds( (gptr)( (const char *)src + 16 * (int64_t)( e + tid ) ),
+                                              (lptr)( (char *)dst + 16 * ( e + first ) ), 16, 0, 0 );
+}
+__device__ __forceinline__ void stage_wait()
+{
+    __builtin_amdgcn_s_waitcnt( 0x0f70 ); // vmcnt( 0 ): the copies have reached LDS
+    __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -1335,96 +1357,118 @@ struct pass_kernel
             constexpr int NH = N / 2 + 1;
             __shared__ int64_t loff[2 * TW], xoff[2 * TW];
             C                 *st = reinterpret_cast<C *>( lds );
-            // 2 TW lines can exceed the thread count (TPC = 1 for N <= 16): strided fill
-            for ( int l = tid; l < 2 * TW; l += NT )
+            // dense rows (every 3D and slab array): the tile is one contiguous piece of the
+            // array, copied into LDS without registers or address arithmetic per bin.  Rows
+            // of 2^26 values in all, before -> with this: FP32 N = 512 111 -> 95 us, 1000
+            // 155 -> 117; FP64 512 215 -> 203, 144 230 -> 203
+            const bool dense = !( IOM & IO_H16_IN ) && p.d0 >= p.ncols && p.ies == 1 && p.is0 == NH &&
+                               ( x.tile + 1 ) * 2 * TW <= p.ncols &&
+                               ( reinterpret_cast<uintptr_t>( p.in ) & 15 ) == 0;
+            if ( dense )
             {
-                const int64_t c  = x.tile * TW * 2 + l;
-                int64_t       io = 0, oo = 0, xi = 0, yo = 0;
-                col_offsets<MG>( p, c < p.ncols ? c : 0, io, oo );
-                if constexpr ( IOM & IO_H16_IN )
-                    col_exponents<MG>( p, c < p.ncols ? c : 0, xi, yo );
-                loff[l] = c < p.ncols ? io : -1;
-                xoff[l] = xi;
+                constexpr int N16 = 2 * TW * NH * (int)sizeof( C ) / 16;
+                stage_copy16( static_cast<const C *>( p.in ) + x.tile * ( 2 * TW * NH ), st, N16, tid, NT );
+                stage_wait();
             }
-            __syncthreads();
-            // every load is issued before the first LDS write, unconditionally (an item
-            // past the end or in a column past the end reads element 0, which exists) and
-            // selected afterwards, so that no load waits on a branch
-            constexpr int ITEMS = 2 * TW * NH;
-            constexpr int PER   = ( ITEMS + NT - 1 ) / NT;
-            C             zs[PER];
-            bool          xrow = false;
-            if constexpr ( IOM & IO_H16_IN )
+            else
             {
-                // FP16 lines whose exponent index runs along the line (xsn = 1) and does not
-                // depend on the fastest batch index (xs0 = 0: the C2R pass of the 3D layout,
-                // bin (x, y, z) of y-line exponent z + x xs2).  When the tile's lines lie in
-                // one batch row they share one row of NH exponents, loaded once per tile as
-                // XD2 dwords into LDS (up to 7 bytes past the row: the work area pads its
-                // exponent arrays), instead of one byte load per bin.  Same values, same
-                // arithmetic.
-                constexpr int       XD2 = ( NH + 3 ) / 4 + 1;
-                __shared__ uint32_t xr2[XD2];
-                const int64_t       c0 = x.tile * TW * 2;
-                xrow = p.xsn == 1 && p.xs0 == 0 && ( reinterpret_cast<uintptr_t>( p.xin ) & 3 ) == 0 &&
-                       c0 + 2 * TW <= p.ncols && c0 % p.d0 + 2 * TW <= p.d0;
-                if ( xrow )
+                // 2 TW lines can exceed the thread count (TPC = 1 for N <= 16): strided fill
+                for ( int l = tid; l < 2 * TW; l += NT )
                 {
-                    const int64_t   xf = xoff[0];
-                    const uint32_t *xw = reinterpret_cast<const uint32_t *>( p.xin );
-                    uint32_t        er = 0;
-                    if ( tid < XD2 )
-                        er = xw[( xf >> 2 ) + tid];
-                    const HE *srch = static_cast<const HE *>( p.in );
-                    HE        raw[PER];
-#pragma unroll
-                    for ( int i = 0; i < PER; ++i )
-                    {
-                        const int e  = tid + i * NT;
-                        const int ec = ITEMS % NT == 0 || e < ITEMS ? e : ITEMS - 1;
-                        raw[i]       = srch[loff[ec / NH] + (int64_t)( ec % NH ) * p.ies];
-                    }
-                    if ( tid < XD2 )
-                        xr2[tid] = er;
-                    __syncthreads();
-                    const uint8_t *xb = reinterpret_cast<const uint8_t *>( xr2 ) + ( xf & 3 );
-#pragma unroll
-                    for ( int i = 0; i < PER; ++i )
-                    {
-                        const int e = tid + i * NT;
-                        if ( ITEMS % NT == 0 || e < ITEMS )
-                            st[e] = h16_decode<SPL>( raw[i], (int8_t)xb[e % NH] ); // line * NH + k == e
-                    }
-                }
-            }
-            if ( !xrow )
-            {
-#pragma unroll
-                for ( int i = 0; i < PER; ++i )
-                {
-                    const int     e    = tid + i * NT;
-                    const bool    in   = ITEMS % NT == 0 || e < ITEMS;
-                    const int     ec   = in ? e : ITEMS - 1;
-                    const int     line = ec / NH, k = ec % NH;
-                    const int64_t lo   = loff[line];
-                    const bool    ok   = in && lo >= 0;
-                    const int64_t src  = ok ? lo + (int64_t)k * p.ies : 0;
-                    C             z;
+                    const int64_t c  = x.tile * TW * 2 + l;
+                    int64_t       io = 0, oo = 0, xi = 0, yo = 0;
+                    col_offsets<MG>( p, c < p.ncols ? c : 0, io, oo );
                     if constexpr ( IOM & IO_H16_IN )
-                        z = h16_load<SPL>( p.in, src, p.xin, ok ? xoff[line] + (int64_t)k * p.xsn : 0 );
-                    else
-                        z = static_cast<const C *>( p.in )[src];
-                    zs[i] = ok ? z : mk<T>( 0, 0 );
+                        col_exponents<MG>( p, c < p.ncols ? c : 0, xi, yo );
+                    loff[l] = c < p.ncols ? io : -1;
+                    xoff[l] = xi;
                 }
-#pragma unroll
-                for ( int i = 0; i < PER; ++i )
+                __syncthreads();
+                // every load is issued before the first LDS write, unconditionally (an item
+                // past the end or in a column past the end reads element 0, which exists) and
+                // selected afterwards, so that no load waits on a branch
+                constexpr int ITEMS = 2 * TW * NH;
+                constexpr int PER   = ( ITEMS + NT - 1 ) / NT;
+                C             zs[PER];
+                bool          xrow = false;
+                if constexpr ( IOM & IO_H16_IN )
                 {
-                    const int e = tid + i * NT;
-                    if ( ITEMS % NT == 0 || e < ITEMS )
-                        st[e] = zs[i]; // line * NH + k == e
+                    // FP16 lines whose exponent index runs along the line (xsn = 1) and does not
+                    // depend on the fastest batch index (xs0 = 0: the C2R pass of the 3D layout,
+                    // bin (x, y, z) of y-line exponent z + x xs2).  When the tile's lines lie in
+                    // one batch row they share one row of NH exponents, loaded once per tile as
+                    // XD2 dwords into LDS (up to 7 bytes past the row: the work area pads its
+                    // exponent arrays), instead of one byte load per bin.  Same values, same
+                    // arithmetic.
+                    constexpr int       XD2 = ( NH + 3 ) / 4 + 1;
+                    __shared__ uint32_t xr2[XD2];
+                    const int64_t       c0 = x.tile * TW * 2;
+                    xrow = p.xsn == 1 && p.xs0 == 0 && ( reinterpret_cast<uintptr_t>( p.xin ) & 3 ) == 0 &&
+                           c0 + 2 * TW <= p.ncols && c0 % p.d0 + 2 * TW <= p.d0;
+                    if ( xrow )
+                    {
+                        const int64_t   xf = xoff[0];
+                        const uint32_t *xw = reinterpret_cast<const uint32_t *>( p.xin );
+                        uint32_t        er = 0;
+                        if ( tid < XD2 )
+                            er = xw[( xf >> 2 ) + tid];
+                        const HE *srch = static_cast<const HE *>( p.in );
+                        HE        raw[PER];
+#pragma unroll
+                        for ( int i = 0; i < PER; ++i )
+                        {
+                            const int e  = tid + i * NT;
+                            const int ec = ITEMS % NT == 0 || e < ITEMS ? e : ITEMS - 1;
+                            raw[i]       = srch[loff[ec / NH] + (int64_t)( ec % NH ) * p.ies];
+                        }
+                        if ( tid < XD2 )
+                            xr2[tid] = er;
+                        __syncthreads();
+                        const uint8_t *xb = reinterpret_cast<const uint8_t *>( xr2 ) + ( xf & 3 );
+#pragma unroll
+                        for ( int i = 0; i < PER; ++i )
+                        {
+                            const int e = tid + i * NT;
+                            if ( ITEMS % NT == 0 || e < ITEMS )
+                                st[e] = h16_decode<SPL>( raw[i], (int8_t)xb[e % NH] ); // line * NH + k == e
+                        }
+                    }
                 }
+                if ( !xrow )
+                {
+                    // FP64 in chunks of 8 loads: all of them at once took up to 206 registers,
+                    // two waves per SIMD
+                    constexpr int CH = sizeof( C ) == 16 && PER > 8 ? 8 : PER;
+                    for ( int i0 = 0; i0 < PER; i0 += CH )
+                    {
+#pragma unroll
+                        for ( int i = 0; i < CH; ++i )
+                        {
+                            const int     e    = tid + ( i0 + i ) * NT;
+                            const bool    in   = ITEMS % NT == 0 && PER % CH == 0 ? true : e < ITEMS;
+                            const int     ec   = in ? e : ITEMS - 1;
+                            const int     line = ec / NH, k = ec % NH;
+                            const int64_t lo   = loff[line];
+                            const bool    ok   = in && lo >= 0;
+                            const int64_t src  = ok ? lo + (int64_t)k * p.ies : 0;
+                            C             z;
+                            if constexpr ( IOM & IO_H16_IN )
+                                z = h16_load<SPL>( p.in, src, p.xin, ok ? xoff[line] + (int64_t)k * p.xsn : 0 );
+                            else
+                                z = static_cast<const C *>( p.in )[src];
+                            zs[i] = ok ? z : mk<T>( 0, 0 );
+                        }
+#pragma unroll
+                        for ( int i = 0; i < CH; ++i )
+                        {
+                            const int e = tid + ( i0 + i ) * NT;
+                            if ( ( ITEMS % NT == 0 && PER % CH == 0 ) || e < ITEMS )
+                                st[e] = zs[i]; // line * NH + k == e
+                        }
+                    }
+                }
+                __syncthreads();
             }
-            __syncthreads();
 #pragma unroll
             for ( int b = 0; b < NB0; ++b )
             {
