@@ -17,7 +17,8 @@
 // Batches of 2^23 complex values, FP32 rows / columns: N = 250 25.5 / 28.1 us (5.3 / 4.8
 // TB/s), N = 1080 26.2 / 33.0 us; FP64 250: 44.9 / 48.4 us (6.0 / 5.6 TB/s).  Its
 // predecessor, one radix per thread and ping-pong LDS buffers with every line transformed
-// column-fastest, took 76 / 75, 60 / 68 and 102 / 101 us.
+// column-fastest, took 76 / 75, 60 / 68 and 102 / 101 us.  With the tile chosen by
+// any_cost, the 175 x 250 x 330 FP32 pair went from 180 (tiles of a fixed size) to 171 us.
 #pragma once
 
 #include "mi_pass.hpp"
@@ -36,9 +37,16 @@ constexpr int any_butterflies( int R, int csize )
     const int n = any_values( csize ) / R;
     return n < 1 ? 1 : ( n > 4 ? 4 : n );
 }
-// Radices of the kernels that most lengths use; a length with a factor 11 or 13 takes the
-// kernels that have those as well (their butterflies need more registers, which the other
-// lengths would pay for in occupancy).
+// The kernels that most lengths use have the common radices and read their twiddles from an
+// LDS copy of the table.  A length with a factor 11 or 13 takes kernels that have every radix
+// (their butterflies need more registers, which the other lengths would pay for in
+// occupancy), one with too large a table kernels that read it from memory.
+enum : int
+{
+    ANY_COMMON = 0,
+    ANY_RARE   = 1,
+    ANY_MEMTW  = 2
+};
 constexpr bool any_common_radix( int R, int csize )
 {
     return R <= 10 || ( csize == 8 && R != 11 && R != 13 && R <= 16 );
@@ -60,14 +68,16 @@ struct any_plan
     int32_t   nt;    // threads (a multiple of cols in column-fastest tiles)
     int32_t   elems; // LDS values of the tile; the twiddle table follows
     int32_t   nh;    // N / 2 + 1
-    int32_t   rare;  // has a radix outside any_common_radix
+    int32_t   mode;  // ANY_COMMON, ANY_RARE or ANY_MEMTW
     uint32_t  mg_n, mg_nh, mg_cols;
     any_stage s[ANY_MAX_STAGES];
 };
 
-template <typename T, int KIND, bool INV, bool LOADB, bool RARE>
+template <typename T, int KIND, bool INV, bool LOADB, int MODE>
 struct any_kernel
 {
+    static constexpr bool RARE = MODE != ANY_COMMON; // every radix
+    static constexpr bool TWL  = MODE != ANY_MEMTW;  // stage twiddles from an LDS copy of the table
     using C                  = cpx<T>;
     static constexpr int CPT = KIND == KIND_C2C ? 1 : 2;
 
@@ -187,30 +197,32 @@ struct any_kernel
                 }
                 else if constexpr ( FIRST )
                 {
-                    // C2R: z = A~ + i B~ from the tile's staged half spectra
+                    // C2R: z = A~ + i B~ from the tile's staged half spectra.  Element n = j + r
+                    // nbf lies below N / 2 for r < R / 2 and is the mirror image of bin N - n
+                    // above; the middle r of an odd radix has both.
+                    const int as = LOADB ? 2 * a.cols : 1, bs = LOADB ? 1 : a.nh;
+                    const C  *at = x.lds + ( LOADB ? 2 * c : 2 * c * a.nh );
+                    const T   h  = p.wmode == 2 ? (T)0.5 : (T)1;
 #pragma unroll
                     for ( int r = 0; r < R; ++r )
                     {
-                        const int n  = j + r * s.nbf;
-                        const int nn = 2 * n <= a.N ? n : a.N - n;
-                        const int at = LOADB ? ( nn << ( a.csh + 1 ) ) + 2 * c : 2 * c * a.nh + nn;
-                        C         za = x.lds[at], zb = x.lds[LOADB ? at + 1 : at + a.nh];
-                        if ( 2 * n > a.N )
+                        const int  n   = j + r * s.nbf;
+                        const bool up  = 2 * r >= R || ( 2 * r + 1 == R && 2 * n > a.N );
+                        const int  nn  = up ? a.N - n : n;
+                        C          za = at[nn * as], zb = at[nn * as + bs];
+                        if ( p.wmode == 2 && n != 0 && 2 * n != a.N )
                         {
-                            za.y = -za.y;
-                            zb.y = -zb.y;
+                            // adjoint of R2C: interior bins carry weight 1/2
+                            za = scl( za, h );
+                            zb = scl( zb, h );
                         }
-                        if ( n == 0 || 2 * n == a.N )
+                        // the imaginary parts of the DC and Nyquist bins are ignored
+                        if ( ( r == 0 && n == 0 ) || ( ( 2 * r == R || 2 * r + 1 == R ) && 2 * n == a.N ) )
                         {
                             za.y = (T)0;
                             zb.y = (T)0;
                         }
-                        else if ( p.wmode == 2 )
-                        {
-                            za = scl( za, (T)0.5 );
-                            zb = scl( zb, (T)0.5 );
-                        }
-                        v[b][r] = mk<T>( za.x - zb.y, za.y + zb.x );
+                        v[b][r] = up ? mk<T>( za.x + zb.y, zb.x - za.y ) : mk<T>( za.x - zb.y, za.y + zb.x );
                     }
                 }
                 else
@@ -221,8 +233,9 @@ struct any_kernel
 #pragma unroll
                     for ( int r = 0; r < R; ++r, at += st )
                         v[b][r] = *at;
-                    const C  *tw = x.tw;
                     const int ts = k * s.tst;
+                    // one kind of pointer per kernel: one that may be either needs slow loads
+                    const C *tw = TWL ? x.tw : p.tw;
 #pragma unroll
                     for ( int r = 1; r < R; ++r )
                     {
@@ -356,6 +369,20 @@ struct any_kernel
         const int             lines = 2 * a.cols;
         const int             items = lines * a.nh;
         constexpr int         U     = 9;
+        if constexpr ( !LOADB )
+        {
+            // dense rows: the tile's half spectra are one contiguous piece of the array (a
+            // whole number of 16-byte pieces, lines is even), copied with no address
+            // arithmetic per bin
+            const C *src = static_cast<const C *>( p.in ) + x.tile * items;
+            if ( p.d0 >= p.ncols && p.ies == 1 && p.is0 == a.nh && ( x.tile + 1 ) * lines <= p.ncols &&
+                 ( reinterpret_cast<uintptr_t>( p.in ) & 15 ) == 0 )
+            {
+                stage_copy16( src, x.lds, items * (int)sizeof( C ) / 16, x.tid, x.nt );
+                stage_wait();
+                return;
+            }
+        }
         for ( int e0 = x.tid; e0 < items; e0 += U * x.nt )
         {
             C    z[U];
@@ -435,7 +462,7 @@ struct any_kernel
             x.c = x.tid & ( a.cols - 1 );
             line_offsets( p, ( x.tile * a.cols + x.c ) * CPT, x.ia, x.ib, x.oa, x.ob, x.va, x.vb );
         }
-        if ( a.nst > 1 )
+        if ( TWL && a.nst > 1 )
             for ( int e = x.tid; e < a.N; e += x.nt )
                 x.tw[e] = p.tw[e];
         if constexpr ( KIND == KIND_C2R )
@@ -461,13 +488,13 @@ struct any_kernel
     }
 };
 
-template <typename T, int KIND, bool INV, bool LOADB, bool RARE>
+template <typename T, int KIND, bool INV, bool LOADB, int MODE>
 __global__ void __launch_bounds__( any_max_threads( 2 * sizeof( T ) ) )
-    __attribute__( ( amdgpu_waves_per_eu( ( sizeof( T ) == 4 ? 6 : 4 ) - ( RARE ? 1 : 0 ) ) ) )
+    __attribute__( ( amdgpu_waves_per_eu( ( sizeof( T ) == 4 ? 6 : 4 ) - ( MODE != ANY_COMMON ? 1 : 0 ) ) ) )
     k_pass_any( const pass_params<T> p, const any_plan a )
 {
     extern __shared__ __align__( 16 ) unsigned char any_lds[];
-    any_kernel<T, KIND, INV, LOADB, RARE>::run( p, a, reinterpret_cast<cpx<T> *>( any_lds ) );
+    any_kernel<T, KIND, INV, LOADB, MODE>::run( p, a, reinterpret_cast<cpx<T> *>( any_lds ) );
 }
 
 } // namespace fftm_mi

@@ -99,40 +99,30 @@ int csize_of( int prec )
     return prec == FFTM_MI_F32 ? 8 : 16;
 }
 
-// The schedule of a runtime-length pass: as few of the kernel's radices as multiply to N.
-// Among those, the first one first by the LDS bank conflicts of stage 0's writes, which have
-// its stride (an odd radix none, twice an odd one two-fold), then the most even ones (the
-// smallest sum).  best.n = 0 if there is none.
+// Schedules of a runtime-length pass: the ways to write N with as few of the kernel's
+// radices as possible, in descending order.
 struct any_schedule
 {
-    int n = 0, cost = 0, r[ANY_MAX_STAGES] = {};
+    int n = 0, r[ANY_MAX_STAGES] = {};
 };
 
-void any_radices( int64_t N, int csize, int maxr, any_schedule cur, any_schedule &best )
+void any_schedules( int64_t N, int csize, int maxr, any_schedule cur, std::vector<any_schedule> &found )
 {
     if ( N == 1 )
     {
-        int first = 0;
-        for ( int i = 1; i < cur.n; ++i )
-            if ( ( cur.r[i] & -cur.r[i] ) < ( cur.r[first] & -cur.r[first] ) )
-                first = i;
-        const int conflict = cur.r[first] & -cur.r[first];
-        std::swap( cur.r[0], cur.r[first] );
-        cur.cost = ( conflict > 2 ? conflict * 100 : 0 );
-        for ( int i = 0; i < cur.n; ++i )
-            cur.cost += cur.r[i];
-        if ( best.n == 0 || cur.n < best.n || ( cur.n == best.n && cur.cost < best.cost ) )
-            best = cur;
+        if ( !found.empty() && cur.n < found[0].n )
+            found.clear();
+        found.push_back( cur );
         return;
     }
-    if ( cur.n == ANY_MAX_STAGES || ( best.n && cur.n == best.n ) )
+    if ( cur.n == ANY_MAX_STAGES || ( !found.empty() && cur.n == found[0].n ) )
         return;
     for ( int r = maxr; r >= 2; --r )
         if ( N % r == 0 && any_radix( r, csize ) )
         {
             any_schedule next = cur;
             next.r[next.n++]  = r;
-            any_radices( N / r, csize, r, next, best );
+            any_schedules( N / r, csize, r, next, found );
         }
 }
 
@@ -141,26 +131,102 @@ uint32_t mulhi_magic( int64_t d )
     return d > 1 ? (uint32_t)( ( ( (uint64_t)1 << 32 ) / (uint64_t)d ) + 1 ) : 0;
 }
 
+// Estimated cost of a tile of `cols` lines of a runtime-length pass with nt threads, lower
+// is better; negative if a stage needs more butterflies per thread than the kernel holds.
+// The terms: lanes idle in some stage (1: none), wavefronts per CU short of 24, octaves off
+// 256 threads, bank conflicts of stage 0's writes (stride r0), bytes in flight per CU short
+// of 128 KB, loads per thread in stage 0, trips per stage, LDS, short rows.  The weights were
+// fitted to 30 000 measured (schedule, cols, nt) of 31 lengths 12..2000 in all kinds, 2^22
+// and 2^25 values: the choice takes 1.03..1.05 times the best measured time there, the
+// fixed-size tiles before it 1.07..1.14.
+double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool loadb, int64_t cols, int nt,
+                 int64_t lines )
+{
+    double slots = 0, trips = 0;
+    for ( int i = 0; i < s.n; ++i )
+    {
+        const int64_t k = ( N / s.r[i] * cols + nt - 1 ) / nt;
+        if ( k > any_butterflies( s.r[i], csize ) )
+            return -1;
+        slots += (double)( k * s.r[i] * nt ) / (double)( N * cols * s.n );
+        trips += (double)k / s.n;
+    }
+    const double lds      = (double)( line * cols * csize + ( N * csize <= 16384 ? N * csize : 0 ) );
+    const int    per_wg   = nt / 64, cap = csize == 8 ? 24 : 20; // wavefronts; registers allow `cap` per CU
+    const int    wgs      = std::max( 1, std::min( (int)( lds_limit_wide_bytes() / lds ), cap / per_wg ) );
+    const double waves    = std::max( 0.0, 1.0 - wgs * per_wg / 24.0 );
+    const double inflight = std::max( 0.0, 1.0 - wgs * (double)( N * cols * csize ) / 131072.0 );
+    const double octaves  = std::abs( std::log2( nt / 256.0 ) );
+    const double first    = s.r[0] / 16.0;
+    const double conflict = std::max( 0, ( s.r[0] & -s.r[0] ) - 2 );
+    const double row      = std::max( 0.0, 1.0 - cols * csize / 128.0 );
+    const double sector   = loadb && cols * csize < 32 ? 10 : 0; // below one only where nothing else fits
+    const double fill     = std::max( 0.0, 2.0 - 2.0 * (double)( ( lines + cols - 1 ) / cols ) / 512.0 );
+    if ( csize == 8 )
+        return loadb ? 1 + sector + fill + 0.8 * slots + 0.8 * waves + 0.1 * octaves + 0.05 * conflict + 0.3 * inflight -
+                           0.8 * first + 0.8 * row
+                     : 1 + fill + 0.8 * slots + 0.8 * waves + 0.1 * octaves + 0.05 * conflict - 0.1 * first + 0.1 * lds / 65536 +
+                           0.1 / 16 * ( (double)( N * cols ) / nt );
+    return loadb ? 1 + sector + fill + 0.8 * slots + 0.5 * octaves + 0.3 * conflict + 0.8 * inflight - 0.3 * first +
+                       0.8 * lds / 65536
+                 : 1 + fill + 0.5 * slots + 0.3 * octaves + 0.05 * conflict - 0.1 * first + 0.3 * trips + 0.8 * lds / 65536;
+}
+
 // Schedule and tile of a runtime-length pass; false if the length is out of range.
-bool make_any_plan( int64_t N, int csize, bool loadb, int kind, any_plan &a )
+bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, any_plan &a )
 {
     a    = any_plan{};
     a.N  = (int32_t)N;
     a.nh = (int32_t)( N / 2 + 1 );
-    any_schedule sch;
+    std::vector<any_schedule> found;
     if ( N == 1 )
-        sch.r[sch.n++] = 1;
+    {
+        found.emplace_back();
+        found[0].n    = 1;
+        found[0].r[0] = 1;
+    }
     else
-        any_radices( N, csize, 16, any_schedule{}, sch );
-    if ( sch.n == 0 )
+        any_schedules( N, csize, 16, any_schedule{}, found );
+    const int64_t line = std::max<int64_t>( N, kind == KIND_C2R ? 2 * a.nh : 0 ); // LDS values per line (pair)
+    const int64_t lines = kind == KIND_C2C ? ncols : ( ncols + 1 ) / 2;
+    double        best = -1;
+    any_schedule  sch;
+    for ( any_schedule s : found )
+        for ( int f = 0; f < s.n; ++f )
+        {
+            // radix f first, the others in descending order
+            if ( f > 0 && s.r[f] == s.r[0] )
+                continue;
+            std::rotate( s.r, s.r + f, s.r + f + 1 );
+            // column-fastest tiles: a power of two of columns; line-fastest: any number of lines
+            for ( int64_t c = 1; c <= 64; c += loadb ? c : std::max<int64_t>( 1, c / 6 ) )
+            {
+                if ( c > 1 && line * c * csize > ( loadb ? 81920 : 45056 ) )
+                    break;
+                // threads that hold about 5 to 16 values each
+                const int64_t v0 = N * c / 16, v1 = N * c / 5;
+                for ( int nt = (int)std::max<int64_t>( 64, v0 / 64 * 64 );
+                      nt <= any_max_threads( csize ) && nt <= v1 + 64; nt += 64 )
+                {
+                    const double v = any_cost( s, N, line, csize, loadb, c, nt, lines );
+                    if ( v >= 0 && ( best < 0 || v < best ) )
+                    {
+                        best   = v;
+                        sch    = s;
+                        a.cols = (int32_t)c;
+                        a.nt   = nt;
+                    }
+                }
+            }
+            std::rotate( s.r, s.r + 1, s.r + f + 1 );
+        }
+    if ( best < 0 )
         return false;
-    int per = any_values( csize ) + 3; // values per thread that whole butterflies of every stage allow
-    a.nst   = sch.n;
+    a.nst      = sch.n;
     int64_t ns = 1;
     for ( int i = 0; i < sch.n; ++i )
     {
         const int r   = sch.r[i];
-        per           = std::min( per, any_butterflies( r, csize ) * r );
         a.s[i].r      = r;
         a.s[i].ns     = (int32_t)ns;
         a.s[i].nbf    = (int32_t)( N / r );
@@ -168,42 +234,52 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, any_plan &a )
         a.s[i].mg_nbf = mulhi_magic( N / r );
         a.s[i].mg_ns  = mulhi_magic( ns );
         if ( r > 1 && !any_common_radix( r, csize ) )
-            a.rare = 1;
+            a.mode = ANY_RARE;
         ns *= r;
     }
-    a.mg_n  = mulhi_magic( N );
-    a.mg_nh = mulhi_magic( a.nh );
-    const int64_t line = std::max<int64_t>( N, kind == KIND_C2R ? 2 * a.nh : 0 ); // LDS values per line (pair)
-    int           cols;
-    if ( loadb )
-    {
-        // one 128-byte row segment, narrower where the tile would not fit 64 KB, wider for
-        // short lines
-        cols = 128 / csize;
-        while ( cols > 1 && ( line * cols * csize > 65536 || N * cols > (int64_t)per * any_max_threads( csize ) ) )
-            cols /= 2;
-        while ( cols < 64 && N * cols / per < 256 && N * cols * csize <= 16384 )
-            cols *= 2;
-        while ( ( 1 << a.csh ) < cols )
-            ++a.csh;
-    }
-    else
-    {
-        cols = (int)std::max<int64_t>( 1, 256 * per / N );
-        while ( cols > 1 && line * cols * csize > 32768 )
-            --cols;
-    }
-    a.cols    = cols;
-    a.mg_cols = mulhi_magic( cols );
-    a.elems   = (int32_t)( line * cols );
-    a.nt      = (int32_t)( ( ( N * cols + per - 1 ) / per + 63 ) / 64 * 64 );
-    return a.nt <= any_max_threads( csize );
+    while ( loadb && ( 1 << a.csh ) < a.cols )
+        ++a.csh;
+    a.mg_n    = mulhi_magic( N );
+    a.mg_nh   = mulhi_magic( a.nh );
+    a.mg_cols = mulhi_magic( a.cols );
+    a.elems   = (int32_t)( line * a.cols );
+    // the LDS copy of the twiddle table up to 16 KB (32 KB cost FP64 2..6 %)
+    if ( a.nst > 1 && N * csize > 16384 )
+        a.mode = ANY_MEMTW;
+    return true;
+}
+
+// Compiled 3/5/7-smooth lengths whose contiguous lines the runtime-length kernel transforms
+// faster, with both measured at 2^22 / 2^26 values (time of the compiled one over its time):
+//   R2C FP32 to 288 points, FP64 to 80: 1.04..2.9 / 1.0..2.9 (the compiled tiles hold few
+//   values per thread there and read 4-byte reals), 0.84..1.2 beyond;
+//   C2C FP32 to 56, FP64 to 144: 0.94..1.7 / 0.97..1.5, beyond that down to 0.7;
+//   FP32 from 1000 points where radices up to 16 save a stage and the odd part is above 15
+//   (1000 = 10 10 10 instead of 8 5 5 5): 1.0..1.5 / 1.0..1.4; 0.8..1.1 for 2^k 3, 5, 9 or 15.
+// C2R lines, and columns, which differ by less and in both directions, stay compiled.
+bool runtime_rows( const pass_rt &p, int csize )
+{
+    if ( p.loadb || pow2_length( p.N ) || p.kind == KIND_C2R )
+        return false;
+    if ( p.N <= ( p.kind == KIND_R2C ? ( csize == 8 ? 288 : 80 ) : ( csize == 8 ? 56 : 144 ) ) )
+        return true;
+    if ( csize != 8 || p.N < 1000 )
+        return false;
+    int64_t odd = p.N;
+    while ( odd % 2 == 0 )
+        odd /= 2;
+    std::vector<any_schedule> found;
+    any_schedules( p.N, csize, 16, any_schedule{}, found );
+    return odd > 15 && !found.empty() && found[0].n < make_rplan( (int)p.N ).n;
 }
 
 // Decide how a pass of length N runs (fixed kernel or generic); fills N-dependent fields.
-int configure_kernel( pass_rt &p, int prec )
+// plan = false: only whether it can run (every 13-smooth length in range has a plan).
+int configure_kernel( pass_rt &p, int prec, bool plan )
 {
-    if ( fixed_supported( p.N ) )
+    if ( fixed_supported( p.N ) &&
+         !( plan && runtime_rows( p, csize_of( prec ) ) &&
+            make_any_plan( p.N, csize_of( prec ), p.loadb, p.kind, p.ncols, p.any ) ) )
     {
         p.generic = false;
         return ok();
@@ -217,7 +293,8 @@ int configure_kernel( pass_rt &p, int prec )
                      "fftm_mi: transform length " + std::to_string( p.N ) +
                          " has a prime factor above 13 (not supported yet)" );
     const int cs = csize_of( prec );
-    if ( 2 * p.N * cs > 65536 || !make_any_plan( p.N, cs, p.loadb, p.kind, p.any ) )
+    if ( ( !fixed_supported( p.N ) && 2 * p.N * cs > 65536 ) ||
+         ( plan && !make_any_plan( p.N, cs, p.loadb, p.kind, p.ncols, p.any ) ) )
         return fail( FFTM_MI_NOT_SUPPORTED,
                      "fftm_mi: transform length " + std::to_string( p.N ) + " exceeds the single-pass limit" );
     p.generic = true;
@@ -544,7 +621,7 @@ int prepare_passes( std::vector<pass_rt> &passes, int prec, tables *tb )
         }
         else if ( !p.plane )
         {
-            const int rc = configure_kernel( p, prec );
+            const int rc = configure_kernel( p, prec, tb != nullptr );
             if ( rc != FFTM_MI_SUCCESS )
                 return rc;
         }
@@ -2507,10 +2584,10 @@ int fftm_mi_ffts_autotune( fftm_mi_ffts h, const void *real_in, void *spectrum_o
             double               best_ms = 1e300;
             int                  best    = cur.var;
             // tile shapes 0..nvar-1, each in every tile order
-            // (plane passes: shape 0 the LDS kernel, 1 the register kernel; any-radix
-            // passes have one shape and their own order)
+            // (plane passes: shape 0 the LDS kernel, 1 the register kernel; runtime-length
+            // passes have one shape)
             const int            nvar    = cur.generic ? 1 : ( cur.plane ? 2 : fixed_variants( cur.N ) );
-            const int            ncand   = cur.generic ? 1 : NUM_ORDERS * nvar;
+            const int            ncand   = NUM_ORDERS * nvar;
             // radix schedules 1 and 2 (alternative schedule, and its radix-16 stage on the
             // matrix cores) where compiled, for passes with FP32 output (their validity is a
             // tolerance against variant 0's output, see below)

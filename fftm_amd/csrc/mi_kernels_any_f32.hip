@@ -15,12 +15,14 @@ hipError_t launch_one( const pass_params<float> &p, const any_plan &a, hipStream
         return hipSuccess;
     if ( ntiles > 0x7fffffffLL )
         return hipErrorInvalidConfiguration;
-    const size_t lds = sizeof( cpx<float> ) * (size_t)( a.elems + ( a.nst > 1 ? a.N : 0 ) );
+    const size_t lds = sizeof( cpx<float> ) * (size_t)( a.elems + ( a.nst > 1 && a.mode != ANY_MEMTW ? a.N : 0 ) );
     const dim3   grid( (unsigned)ntiles ), block( (unsigned)a.nt );
-    if ( a.rare )
-        hipLaunchKernelGGL( ( k_pass_any<float, KIND, INV, LOADB, true> ), grid, block, lds, s, p, a );
+    if ( a.mode == ANY_MEMTW )
+        hipLaunchKernelGGL( ( k_pass_any<float, KIND, INV, LOADB, ANY_MEMTW> ), grid, block, lds, s, p, a );
+    else if ( a.mode == ANY_RARE )
+        hipLaunchKernelGGL( ( k_pass_any<float, KIND, INV, LOADB, ANY_RARE> ), grid, block, lds, s, p, a );
     else
-        hipLaunchKernelGGL( ( k_pass_any<float, KIND, INV, LOADB, false> ), grid, block, lds, s, p, a );
+        hipLaunchKernelGGL( ( k_pass_any<float, KIND, INV, LOADB, ANY_COMMON> ), grid, block, lds, s, p, a );
     return hipGetLastError();
 }
 

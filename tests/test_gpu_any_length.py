@@ -9,10 +9,11 @@ import pytest
 
 from helpers import check_close, from_gpu, to_gpu
 
-# 1..15: single stages; 3125 = 5^5 five stages; primes 11 and 13 alone, squared and cubed;
+# compiled lengths whose rows take the runtime kernel (12, 20, 48, 56, 100, 144, 1000, 1680)
+# and others; 1..15: single stages; 3125 = 5^5 five stages; primes 11 and 13 alone, squared and cubed;
 # the largest lengths each precision takes
-LENGTHS = [1, 3, 6, 7, 9, 11, 13, 14, 15, 18, 22, 26, 39, 45, 99, 125, 143, 169, 175, 234, 250, 330, 343, 420, 625, 720,
-           1001, 1080, 1331, 2016, 2197, 3125, 3993, 4004, 4095]
+LENGTHS = [1, 3, 6, 7, 9, 11, 12, 13, 14, 15, 18, 20, 22, 26, 39, 45, 48, 56, 99, 100, 125, 143, 144, 169, 175, 234, 250, 330, 343, 420, 625, 720,
+           1000, 1001, 1080, 1331, 1680, 2016, 2197, 3125, 3993, 4004, 4095]
 MAX_LENGTH = {"float32": 4096, "float64": 2048}
 
 
