@@ -578,13 +578,73 @@ int run_passes( const std::vector<pass_rt> &passes, const tables &tb, int prec, 
 
 // Default tile order of a new pass: chunks of 32 tiles per XCD (order 3) where the pass
 // has enough work for every XCD to run several chunks, else one contiguous range per
-// XCD (order 0).  Measured with the default shapes: 512^3 pair 1517 -> 1333 us, 256^3
+// XCD (order 0), or round-robin (order 1) for the workgroups of a plane pass, which share
+// nothing.  Measured with the default shapes: 512^3 pair 1517 -> 1333 us, 256^3
 // 177 -> 168 us, 128^4 2653 -> 2585 us; below ~2000 tiles (64^3, 128^3) order 0 is
-// 2-6 % faster.  The tuner times every order regardless.
+// 2-6 % faster; plane passes of 128^3 FP32 13.0 -> 12.7 us, FP64 18.4 -> 17.5 us in order 1.
+// The tuner times every order regardless.
 int default_order( const pass_rt &p )
 {
-    const bool big = p.plane ? p.nplanes >= 2048 : p.ncols >= 32768;
-    return big ? 3 : 0;
+    if ( p.plane )
+        return p.nplanes >= 2048 ? 3 : 1;
+    return p.ncols >= 32768 ? 3 : 0;
+}
+
+// Default tile shape of a new pass (pick_geom's variants; the tuner times all of them).
+// Microseconds per pass in the default order, shape 0 against the one taken, over arrays
+// on both sides of what the 256 MB memory-side cache holds with input and output:
+//   columns, N = 512: twice the threads per column (2): 512^3 FP32 y 204 -> 188, x 206 ->
+//     200, FP64 414 -> 400, 414 -> 411;
+//   columns, N >= 1024 (a 128-byte row segment of them is 128 KB and more): split exchange
+//     with full row segments (3): 1024 x 1024 x 256 FP32 x 943 -> 534, y 496 -> 454, FP64
+//     1024 x 512 x 256 885 -> 577; FP32 arrays that the cache holds are 2-15 % better off
+//     with 2 (1024 x 128 x 128 31.9 -> 29.0 against 34.0) up to N = 2048;
+//   columns, N = 256: 3 beyond the cache (256 x 1024 x 512 FP32 221 -> 193, 256^3 FP64 49.0
+//     -> 46.8), level with 0 and 2 within it for FP32 and 13 % slower;
+//   columns, N = 128, FP64: split exchange (6), 64 x 128 x 1024 26.2 -> 24.1;
+//   FP32 real rows, N = 64 and 256: 2 (R2C 12.6 -> 11.5, 27.0 -> 26.3; C2R 13.6 -> 12.3, 27.4
+//     -> 26.2), N = 128 R2C: 6 within the cache (27.7 -> 25.6), 5 beyond it (431 -> 403);
+//   FP16-stored columns: 6 where FP16 lines are read (512^3 157 -> 141, 197 -> 188, 177 ->
+//     164; shape 7 before: 192, 254, 246), 2 where they are only written or N >= 1024;
+//   hi + lo storage: 6 below N = 512, 2 from there (105 against 115); FP16-reading C2R: 2.
+int default_shape( const pass_rt &p, int csize )
+{
+    if ( p.plane || p.generic || !pow2_length( p.N ) || p.N < 64 )
+        return p.plane ? variant_shape_of( p.var ) : 0;
+    if ( p.iom )
+    {
+        if ( p.kind != KIND_C2C )
+            return p.kind == KIND_C2R && !p.loadb && p.N <= 512 ? 2 : 0;
+        if ( p.iom & IO_SPLIT )
+            return p.loadb ? ( p.N < 512 ? 6 : 2 ) : 0;
+        return p.loadb ? ( ( p.iom & IO_H16_IN ) && p.N < 1024 ? 6 : 2 ) : 0;
+    }
+    const int64_t bytes  = p.ncols * p.N * csize / ( p.kind == KIND_C2C ? 1 : 2 );
+    const bool    beyond = 2 * bytes > (int64_t)256 << 20;
+    if ( p.kind != KIND_C2C )
+    {
+        if ( csize != 8 || p.loadb )
+            return 0;
+        if ( p.N == 128 && p.kind == KIND_R2C )
+            return beyond ? 5 : 6;
+        return p.N == 64 || p.N == 256 ? 2 : 0;
+    }
+    if ( !p.loadb )
+        return 0;
+    if ( csize == 8 )
+        return p.N < 256 ? 0 : ( p.N == 256 ? ( beyond ? 3 : 2 ) : ( p.N >= 4096 || ( p.N >= 1024 && beyond ) ? 3 : 2 ) );
+    return p.N >= 1024 ? 3 : ( p.N == 512 ? 2 : ( p.N == 256 ? ( beyond ? 3 : 0 ) : ( p.N == 128 ? 6 : 0 ) ) );
+}
+
+// Default tile shape of the fused filter pass (shapes 0, 2, 4): twice the threads per
+// column (2), 512^3 Poisson FP32 1111 -> 1043 us, FP64 2116 -> 2052, 1024 x 128 x 128 FP32
+// 137 -> 116, level or better everywhere else but for FP64 tiles of 64-byte rows: twice the
+// columns (4) for N >= 2048 (2048 x 128 x 64 355 -> 310, 4096 x 64 x 64 256 -> 251 against
+// 302) and for N = 1024 beyond the cache (1024 x 512 x 256 2671 -> 2390).
+int default_filter_shape( const pass_rt &p, int csize )
+{
+    const bool beyond = 2 * p.ncols * p.N * csize > (int64_t)256 << 20;
+    return csize == 16 && ( p.N >= 2048 || ( p.N == 1024 && beyond ) ) ? 4 : 2;
 }
 
 // a variant number this pass can run: FP16-storage passes have tile shapes 0, 2, 6, 7; the
@@ -606,8 +666,6 @@ bool pass_variant_ok( const pass_rt &r, int var, int prec )
 int prepare_passes( std::vector<pass_rt> &passes, int prec, tables *tb )
 {
     for ( pass_rt &p : passes )
-        p.var = variant_shape_of( p.var ) + 8 * default_order( p );
-    for ( pass_rt &p : passes )
     {
         if ( p.iom )
         {
@@ -625,6 +683,7 @@ int prepare_passes( std::vector<pass_rt> &passes, int prec, tables *tb )
             if ( rc != FFTM_MI_SUCCESS )
                 return rc;
         }
+        p.var = default_shape( p, csize_of( prec ) ) + 8 * default_order( p );
         if ( tb )
         {
             int rt = tb->ensure( p.N );
@@ -914,9 +973,6 @@ pass_rt axis_pass_h16( int kind, bool inv, int ax, int dim, const int64_t *ext, 
         if ( k != ax )
             v.push_back( bdim{ ext[k], si[k], so[k], xs ? xs[k] : 0, ys ? ys[k] : 0 } );
     rc = set_batch( p, v );
-    // strided lines: twice the columns per workgroup (FP16 rows of 128 bytes), split exchange
-    // (hi + lo storage: 8-byte bins, the split exchange at the default tile)
-    p.var = p.loadb ? ( split ? 6 : 7 ) : 0;
     return p;
 }
 
@@ -2001,12 +2057,14 @@ int ensure_filter_chain( fftm_mi_ffts_s &h )
                          lf.src == BUF_WORK && lf.dst == BUF_WORK && fb.dst == BUF_WORK;
     if ( fusable )
     {
-        // the tile shape follows the tuned forward pass it replaces (shapes 0, 2, 4)
+        // the tile shape follows the forward pass it replaces where that was set to another
+        // than its default (shapes 0, 2, 4), the order always
         pre.back().filter = true;
+        const int cs      = csize_of( h.prec );
         const int lv      = variant_shape_of( lf.var );
-        pre.back().var    = h.flt_var >= 0 ? h.flt_var
-                                           : ( ( lv == 2 || lv == 4 ) ? lv : ( ( lv == 3 || lv == 5 ) ? 4 : 0 ) ) |
-                                                 ( lf.var & ( 3 << 3 ) );
+        const int shape   = lv == default_shape( lf, cs ) ? default_filter_shape( lf, cs )
+                                                          : ( ( lv == 2 || lv == 4 ) ? lv : ( ( lv == 3 || lv == 5 ) ? 4 : 0 ) );
+        pre.back().var    = h.flt_var >= 0 ? h.flt_var : shape | ( lf.var & ( 3 << 3 ) );
         post.erase( post.begin() );
     }
     h.flt_pre     = pre;
