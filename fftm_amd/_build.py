@@ -25,7 +25,7 @@ SOURCES = ["mi_kernels_f32_a.hip", "mi_kernels_f32_b.hip", "mi_kernels_f32_c.hip
            "mi_kernels_filter_f32.hip",
            "mi_kernels_filter_f64.hip",
            "mi_kernels_any_f32.hip", "mi_kernels_any_f64.hip",
-           "mi_kernels_dispatch.hip", "mi_kernels_plane.hip", "mi_host.hip"]
+           "mi_kernels_dispatch.hip", "mi_kernels_plane.hip", "mi_kernels_volume.hip", "mi_host.hip"]
 
 # Packed FP32 VALU ops are disabled for every HIP translation unit (device side).
 HIPFLAGS = [

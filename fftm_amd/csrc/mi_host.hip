@@ -82,6 +82,9 @@ struct pass_rt
     int        iom      = 0;
     int64_t    xsn = 0, xs0 = 0, xs1 = 0, xs2 = 0, ys0 = 0, ys1 = 0, ys2 = 0;
     int64_t    xoff = 0, yoff = 0;
+    // volume pass (the whole transform in one workgroup; generic is set as well)
+    bool       volume   = false;
+    vol_geom   vol{};
     // plane pass (the real axis A of length N and axis B of length NB together)
     bool       plane    = false;
     int64_t    NB       = 0;
@@ -441,6 +444,22 @@ hipError_t launch_plane_one( const pass_rt &r, const tables &tb, const void *src
         return rx ? launch_plane_rx_f64( p, (int)r.N, fwd, s ) : launch_plane_f64( p, (int)r.N, (int)r.NB, fwd, s );
 }
 
+template <typename T>
+hipError_t launch_volume_one( const pass_rt &r, const tables &tb, const void *src, void *dst, hipStream_t s )
+{
+    vol_params<T> p;
+    static_cast<vol_geom &>( p ) = r.vol;
+    p.in    = src;
+    p.out   = dst;
+    p.wmode = r.wmode;
+    for ( int i = 0; i < 4; ++i )
+        p.twg[i] = r.vol.ax[i].nst > 1 ? static_cast<const cpx<T> *>( tb.by_n.at( r.vol.ax[i].n ) ) : nullptr;
+    if constexpr ( std::is_same<T, float>::value )
+        return launch_volume_f32( p, r.kind == KIND_R2C, s );
+    else
+        return launch_volume_f64( p, r.kind == KIND_R2C, s );
+}
+
 // Paired accesses (two consecutive elements per load / store) need unit element stride,
 // a 16-byte aligned base and an even element offset for every line start.
 bool even_line_offsets( const pass_rt &r, int64_t s0, int64_t s1, int64_t s2 )
@@ -478,6 +497,8 @@ template <typename T>
 hipError_t launch_one( const pass_rt &r, const tables &tb, const void *src, void *dst, hipStream_t s,
                        void *work = nullptr, const void *filter = nullptr )
 {
+    if ( r.volume )
+        return launch_volume_one<T>( r, tb, src, dst, s );
     if ( r.plane )
         return launch_plane_one<T>( r, tb, src, dst, s );
     pass_params<T> p{};
@@ -677,7 +698,7 @@ int prepare_passes( std::vector<pass_rt> &passes, int prec, tables *tb )
                                                           "128..2048, got " + std::to_string( p.N ) );
             p.generic = false;
         }
-        else if ( !p.plane )
+        else if ( !p.plane && !p.volume )
         {
             const int rc = configure_kernel( p, prec, tb != nullptr );
             if ( rc != FFTM_MI_SUCCESS )
@@ -687,6 +708,9 @@ int prepare_passes( std::vector<pass_rt> &passes, int prec, tables *tb )
         if ( tb )
         {
             int rt = tb->ensure( p.N );
+            for ( int i = 0; i < 4 && p.volume; ++i )
+                if ( rt == FFTM_MI_SUCCESS && p.vol.ax[i].nst > 1 )
+                    rt = tb->ensure( p.vol.ax[i].n );
             if ( rt == FFTM_MI_SUCCESS && p.plane )
                 rt = tb->ensure( p.NB );
             if ( rt != FFTM_MI_SUCCESS )
@@ -1121,6 +1145,106 @@ void fuse_plane( const ffts_layout &L, int32_t layout, int prec, std::vector<pas
     b.push_back( pb );
     fwd.swap( f );
     bwd.swap( b );
+}
+
+// Replace all passes by one volume pass where the array is small enough for the LDS of one
+// workgroup and for one workgroup to be faster than a launch per axis.
+void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std::vector<pass_rt> &bwd )
+{
+    const int d = L.dim, csize = csize_of( prec );
+    pass_rt   p;
+    vol_geom &v    = p.vol;
+    int64_t   rows = 1;
+    for ( int k = 0; k + 1 < d; ++k )
+        rows *= L.n[k];
+    const int64_t nz = L.n[d - 1];
+    // one workgroup takes 7 us a direction for a few points and 12 for 4096; a launch per
+    // axis takes 13 (3D) and 17 us (4D) throughout: level at about 5500 points, 8000 in 4D
+    if ( nz < 2 || rows < 2 || rows * nz > 1536 * d )
+        return;
+    v.nz    = (int32_t)nz;
+    v.nh    = (int32_t)( nz / 2 + 1 );
+    v.rows  = (int32_t)rows;
+    v.pairs = (int32_t)( ( rows + 1 ) / 2 );
+    v.elems = std::max( v.rows * v.nh, v.pairs * v.nz );
+    int     most = 1; // butterflies of the largest stage
+    int32_t st   = v.nh;
+    for ( int i = 3; i >= 0; --i )
+    {
+        // logical axes at the end: d = 3 has no o0
+        const int     k = i - ( 4 - d );
+        const int64_t n = k < 0 ? 1 : L.n[k];
+        vol_axis     &a = v.ax[i];
+        a.n             = (int32_t)n;
+        v.sr[i]         = k < 0 ? 0 : (int32_t)L.sr[k];
+        v.sc[i]         = k < 0 ? 0 : (int32_t)L.sc[k];
+        a.gs            = i < 3 ? v.sc[i] : v.sr[i];
+        if ( i < 3 )
+        {
+            v.ext[i] = (int32_t)n;
+            a.st     = st;
+            a.rst    = st / v.nh;
+            a.mg_st  = mulhi_magic( st );
+            st *= (int32_t)n;
+        }
+        if ( n == 1 )
+            continue;
+        a.lines    = i < 3 ? v.rows * v.nh / (int32_t)n : v.pairs;
+        a.mg_lines = mulhi_magic( a.lines );
+        std::vector<any_schedule> found;
+        any_schedules( n, 8, 16, any_schedule{}, found ); // every radix up to 16
+        if ( found.empty() || found[0].n > VOL_MAX_STAGES )
+            return;
+        const any_schedule *best = &found[0]; // the most even one
+        for ( const any_schedule &s : found )
+            if ( s.r[0] < best->r[0] )
+                best = &s;
+        a.nst      = best->n;
+        int32_t ns = 1;
+        for ( int t = 0; t < a.nst; ++t )
+        {
+            a.r[t]      = best->r[t];
+            a.mg_ns[t]  = mulhi_magic( ns );
+            a.mg_nbf[t] = mulhi_magic( n / best->r[t] );
+            ns *= best->r[t];
+            a.tst[t] = (int32_t)n / ns;
+            most = std::max( most, ( i < 3 ? v.rows * v.nh : v.pairs * v.nz ) / best->r[t] );
+        }
+        if ( a.nst > 1 )
+        {
+            a.tw = v.twelems;
+            v.twelems += a.n;
+        }
+    }
+    if ( ( 2 * v.elems + v.twelems ) * csize > vol_lds_limit() )
+        return;
+    // forward: real axis, o2, o1, o0; backward the other way round (there the real axis's
+    // first stage always builds its lines from the half spectra)
+    int lo = 0, hi = 2; // first and last complex axis with stages (rows >= 2: there is one)
+    while ( v.ax[lo].nst == 0 )
+        ++lo;
+    while ( v.ax[hi].nst == 0 )
+        --hi;
+    v.ax[3].ffwd = VOL_READ;
+    v.ax[hi].ffwd |= VOL_SEP;
+    v.ax[lo].ffwd |= VOL_WRITE;
+    v.ax[lo].fbwd = VOL_READ;
+    v.ax[3].fbwd  = VOL_READ | VOL_WRITE;
+    v.mg_nh = mulhi_magic( v.nh );
+    v.mg_e1 = mulhi_magic( v.ext[1] );
+    v.mg_e2 = mulhi_magic( v.ext[2] );
+    v.nt    = std::min( ( most + 63 ) / 64 * 64, vol_max_threads( csize ) );
+    p.volume = p.generic = true;
+    p.N      = nz;
+    p.ncols  = rows;
+    p.kind   = KIND_R2C;
+    p.src    = BUF_IN;
+    p.dst    = BUF_OUT;
+    pass_rt q = p;
+    q.kind    = KIND_C2R;
+    q.inv     = true;
+    fwd.assign( 1, p );
+    bwd.assign( 1, q );
 }
 
 int build_ffts_passes( const ffts_layout &L, bool overwrite, std::vector<pass_rt> &fwd, std::vector<pass_rt> &bwd,
@@ -1684,7 +1808,10 @@ int fftm_mi_ffts_validate( int32_t layout, const int64_t *n, int32_t precision, 
     if ( rc != FFTM_MI_SUCCESS )
         return rc;
     if ( !( flags & FFTM_MI_FLAG_NO_PLANE_FUSION ) )
+    {
         fuse_plane( L, layout, precision, f, b );
+        fuse_volume( L, precision, f, b );
+    }
     rc = prepare_passes( f, precision, nullptr );
     if ( rc == FFTM_MI_SUCCESS )
         rc = prepare_passes( b, precision, nullptr );
@@ -1729,7 +1856,10 @@ int fftm_mi_ffts_create( int32_t layout, const int64_t *n, int32_t precision, in
         int64_t we = 0;
         build_ffts_passes( L, ( flags & FFTM_MI_FLAG_OVERWRITE_INPUT ) != 0, p->fwd, p->bwd, we );
         if ( !( flags & FFTM_MI_FLAG_NO_PLANE_FUSION ) )
+        {
             fuse_plane( L, layout, precision, p->fwd, p->bwd );
+            fuse_volume( L, precision, p->fwd, p->bwd );
+        }
     }
     rc = prepare_passes( p->fwd, p->prec, &p->tb );
     if ( rc == FFTM_MI_SUCCESS )
@@ -1859,7 +1989,9 @@ int fftm_mi_ffts_pass_bytes( fftm_mi_ffts h, int32_t backward, int32_t index, in
             *bytes = p.ncols * ( nh * ic + p.N * rs ) + ex;
         return ok();
     }
-    if ( p.plane )
+    if ( p.volume )
+        *bytes = p.vol.rows * ( p.N * rs + nh * cs );
+    else if ( p.plane )
         *bytes = p.nplanes * p.NB * ( p.N * rs + nh * cs );
     else if ( p.kind == KIND_C2C )
         *bytes = 2 * p.ncols * p.N * cs;
@@ -2645,7 +2777,7 @@ int fftm_mi_ffts_autotune( fftm_mi_ffts h, const void *real_in, void *spectrum_o
             // (plane passes: shape 0 the LDS kernel, 1 the register kernel; runtime-length
             // passes have one shape)
             const int            nvar    = cur.generic ? 1 : ( cur.plane ? 2 : fixed_variants( cur.N ) );
-            const int            ncand   = NUM_ORDERS * nvar;
+            const int            ncand   = cur.volume ? 1 : NUM_ORDERS * nvar;
             // radix schedules 1 and 2 (alternative schedule, and its radix-16 stage on the
             // matrix cores) where compiled, for passes with FP32 output (their validity is a
             // tolerance against variant 0's output, see below)

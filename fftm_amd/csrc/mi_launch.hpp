@@ -8,6 +8,7 @@
 #include "mi_any.hpp"
 #include "mi_pass.hpp"
 #include "mi_plane.hpp"
+#include "mi_volume.hpp"
 
 namespace fftm_mi
 {
@@ -85,6 +86,10 @@ hipError_t launch_filter_f32( const pass_params<float> &p, const filter_params<f
                               hipStream_t s );
 hipError_t launch_filter_f64( const pass_params<double> &p, const filter_params<double> &f, int N, bool loadb, int var,
                               hipStream_t s );
+
+// a whole small transform in one workgroup (mi_volume.hpp)
+hipError_t launch_volume_f32( const vol_params<float> &p, bool fwd, hipStream_t s );
+hipError_t launch_volume_f64( const vol_params<double> &p, bool fwd, hipStream_t s );
 
 // lengths without a compiled kernel (mi_any.hpp)
 hipError_t launch_any_f32( const pass_params<float> &p, const any_plan &a, int kind, bool inv, bool loadb, hipStream_t s );
