@@ -150,18 +150,18 @@ struct filter_params
 // floor(S |k| / kmax) evaluated exactly, clamped to S - 1.  Integer arithmetic: on bins
 // where S |k| / kmax is an integer (|k|^2 = 3 on a 6^3 cube with S = 3) a floating
 // floor(sqrt(k2) * S / kmax) can land one shell low.  S <= 1024 and k2, kmax2 < 2^25 keep
-// every product below 2^46.
+// every product below 2^46.  The floating estimate is some ulps of FP32 off a value of at
+// most about 1024, so within one of the answer: one step either way.  (With an FP64 square
+// root and division and two steps either way, the shell index was half of the 256^3 fused
+// filter pass: 62 us, 38 without; the training step with it 588 -> 564 us.)
 __device__ __forceinline__ int shell_of( int64_t k2, int S, int64_t kmax2 )
 {
-    const int64_t rhs = (int64_t)S * S * k2;
-    int           s   = (int)sqrt( (double)rhs / (double)kmax2 ); // within one of the answer
-#pragma unroll
-    for ( int i = 0; i < 2; ++i )
-        s = ( s > 0 && (int64_t)s * s * kmax2 > rhs ) ? s - 1 : s;
-#pragma unroll
-    for ( int i = 0; i < 2; ++i )
-        s = ( (int64_t)( s + 1 ) * ( s + 1 ) * kmax2 <= rhs ) ? s + 1 : s;
-    return s < S - 1 ? s : S - 1;
+    const uint64_t rhs = (uint64_t)( (uint32_t)S * (uint32_t)S ) * (uint32_t)k2;
+    const float    est = (float)S * __builtin_amdgcn_sqrtf( (float)(uint32_t)k2 ) * __builtin_amdgcn_rsqf( (float)(uint32_t)kmax2 );
+    uint32_t       s   = (uint32_t)est;
+    s = (uint64_t)( s * s ) * (uint32_t)kmax2 > rhs ? s - 1 : s; // 0 stays
+    s = (uint64_t)( ( s + 1 ) * ( s + 1 ) ) * (uint32_t)kmax2 <= rhs ? s + 1 : s;
+    return (int)s < S - 1 ? (int)s : S - 1;
 }
 
 // wavenumbers of the bin at spectrum offset off: returns sum_a k_a^2 and sets kd to the
@@ -186,25 +186,44 @@ __device__ __forceinline__ float filter_k2( const filter_params<T> &f, int64_t o
     return k2;
 }
 
-// H(k) as (real, imaginary) parts
-template <typename T>
+// H(k) of operator KIND as (real, imaginary) parts
+template <int KIND, typename T>
 __device__ __forceinline__ cpx<T> filter_h( const filter_params<T> &f, float k2, float kd )
 {
-    switch ( f.kind )
+    if constexpr ( KIND == OP_POISSON )
+        return mk<T>( k2 == 0.f ? (T)0 : (T)( -f.scale ) / (T)k2, (T)0 );
+    else if constexpr ( KIND == OP_GAUSSIAN )
     {
-    case OP_POISSON: return mk<T>( k2 == 0.f ? (T)0 : (T)( -f.scale ) / (T)k2, (T)0 );
-    case OP_GAUSSIAN:
         if constexpr ( sizeof( T ) == 4 )
             return mk<T>( (T)f.scale * __expf( -k2 * (float)f.inv_two_sigma2 ), (T)0 );
         else
             return mk<T>( (T)( f.scale * exp( -(double)k2 * f.inv_two_sigma2 ) ), (T)0 );
-    case OP_DERIVATIVE: return mk<T>( (T)0, (T)f.scale * (T)kd );
-    case OP_POISSON_GRAD: return mk<T>( (T)0, k2 == 0.f ? (T)0 : (T)( -f.scale ) * (T)kd / (T)k2 );
-    case OP_BANDPASS:
+    }
+    else if constexpr ( KIND == OP_DERIVATIVE )
+        return mk<T>( (T)0, (T)f.scale * (T)kd );
+    else if constexpr ( KIND == OP_POISSON_GRAD )
+        return mk<T>( (T)0, k2 == 0.f ? (T)0 : (T)( -f.scale ) * (T)kd / (T)k2 );
+    else if constexpr ( KIND == OP_BANDPASS )
         return mk<T>( ( (double)k2 >= f.klo2 && (double)k2 <= f.khi2 ) ? (T)f.scale : (T)0, (T)0 );
-    default:
+    else
         // k2 is a sum of squared integers below 2^24, exact in FP32
         return mk<T>( (T)f.scale * f.coeffs[shell_of( (int64_t)k2, f.nshells, f.kmax2 )], (T)0 );
+}
+
+// body( KIND ) for the operator's kind, a compile-time constant: one branch for all of a
+// thread's bins instead of one per bin (512^3 FP32 Poisson solve 1039 -> 1013 us, three FP64
+// derivatives of 192 x 160 x 144 with their transforms 247 -> 243)
+template <typename T, typename F>
+__device__ __forceinline__ void with_filter_kind( const filter_params<T> &f, F &&body )
+{
+    switch ( f.kind )
+    {
+    case OP_POISSON: body( std::integral_constant<int, OP_POISSON>{} ); break;
+    case OP_GAUSSIAN: body( std::integral_constant<int, OP_GAUSSIAN>{} ); break;
+    case OP_DERIVATIVE: body( std::integral_constant<int, OP_DERIVATIVE>{} ); break;
+    case OP_POISSON_GRAD: body( std::integral_constant<int, OP_POISSON_GRAD>{} ); break;
+    case OP_BANDPASS: body( std::integral_constant<int, OP_BANDPASS>{} ); break;
+    default: body( std::integral_constant<int, OP_SHELL>{} ); break;
     }
 }
 
@@ -898,24 +917,26 @@ struct pass_kernel
             float       kdc = 0.f;
             const float k2c = filter_k2( *x.f, x.oa, kdc );
             const bool  dline = x.f->dax == x.f->line_m;
+            with_filter_kind( *x.f, [&]( auto op ) {
 #pragma unroll
-            for ( int b = 0; b < NB; ++b )
-            {
-                const int j = jmap<RP.n - 1>( x.t, b );
-                if ( NBF % TPC == 0 || j < NBF )
+                for ( int b = 0; b < NB; ++b )
                 {
-                    const int d = ( j / NS ) * NS * R + ( j % NS );
-#pragma unroll
-                    for ( int m = 0; m < R; ++m )
+                    const int j = jmap<RP.n - 1>( x.t, b );
+                    if ( NBF % TPC == 0 || j < NBF )
                     {
-                        const int n  = d + m * NS;
-                        const int kk = n <= N / 2 ? n : n - N;
-                        v[b][m]      = apply_h( v[b][m],
-                                                filter_h( *x.f, k2c + (float)( kk * kk ), dline ? (float)kk : kdc ),
-                                                x.f->kind );
+                        const int d = ( j / NS ) * NS * R + ( j % NS );
+#pragma unroll
+                        for ( int m = 0; m < R; ++m )
+                        {
+                            const int n  = d + m * NS;
+                            const int kk = n <= N / 2 ? n : n - N;
+                            v[b][m]      = apply_h( v[b][m],
+                                                    filter_h<op()>( *x.f, k2c + (float)( kk * kk ), dline ? (float)kk : kdc ),
+                                                    op() );
+                        }
                     }
                 }
-            }
+            } );
             put_stage<2, RP.n - 1, R, NS, NB>( v, x );
             __syncthreads();
             pass_kernel<T, N, KIND_C2C, true, LOADB, VAR, IO_F32, false>::run_from_lds( x );

@@ -181,10 +181,12 @@ __global__ void __launch_bounds__( 256 )
 #pragma unroll
         for ( int u = 0; u < 4; ++u )
             z[u] = in[o[u] < w.total ? o[u] : o[0]];
+        with_filter_kind( f, [&]( auto op ) {
 #pragma unroll
-        for ( int u = 0; u < 4; ++u )
-            if ( o[u] < w.total )
-                out[o[u]] = apply_h( z[u], filter_h( f, (float)k2[u], (float)kd[u] ), f.kind );
+            for ( int u = 0; u < 4; ++u )
+                if ( o[u] < w.total )
+                    out[o[u]] = apply_h( z[u], filter_h<op()>( f, (float)k2[u], (float)kd[u] ), op() );
+        } );
     } );
 }
 
