@@ -82,7 +82,8 @@ struct pass_rt
     int        iom      = 0;
     int64_t    xsn = 0, xs0 = 0, xs1 = 0, xs2 = 0, ys0 = 0, ys1 = 0, ys2 = 0;
     int64_t    xoff = 0, yoff = 0;
-    // volume pass (the whole transform in one workgroup; generic is set as well)
+    // volume pass (the whole transform, or the planes of its two inner axes, one workgroup
+    // each; generic is set as well)
     bool       volume   = false;
     vol_geom   vol{};
     // plane pass (the real axis A of length N and axis B of length NB together)
@@ -1147,37 +1148,35 @@ void fuse_plane( const ffts_layout &L, int32_t layout, int prec, std::vector<pas
     bwd.swap( b );
 }
 
-// Replace all passes by one volume pass where the array is small enough for the LDS of one
-// workgroup and for one workgroup to be faster than a launch per axis.
-void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std::vector<pass_rt> &bwd )
+// A tile of complex axes first..last (at most three) and the real axis.  False where a length
+// has no schedule or the tile does not fit.
+bool make_tile( const ffts_layout &L, int csize, int first, int last, vol_geom &v )
 {
-    const int d = L.dim, csize = csize_of( prec );
-    pass_rt   p;
-    vol_geom &v    = p.vol;
-    int64_t   rows = 1;
-    for ( int k = 0; k + 1 < d; ++k )
+    const int d    = L.dim;
+    v              = vol_geom{};
+    int64_t rows   = 1;
+    for ( int k = first; k <= last; ++k )
         rows *= L.n[k];
-    const int64_t nz = L.n[d - 1];
-    // one workgroup takes 7 us a direction for a few points and 12 for 4096; a launch per
-    // axis takes 13 (3D) and 17 us (4D) throughout: level at about 5500 points, 8000 in 4D
-    if ( nz < 2 || rows < 2 || rows * nz > 1536 * d )
-        return;
+    const int64_t nz = L.n[d - 1], nh = nz / 2 + 1;
+    if ( std::max( rows * nh, ( rows + 1 ) / 2 * nz ) * 2 * csize > vol_lds_limit() )
+        return false;
     v.nz    = (int32_t)nz;
-    v.nh    = (int32_t)( nz / 2 + 1 );
+    v.nh    = (int32_t)nh;
     v.rows  = (int32_t)rows;
     v.pairs = (int32_t)( ( rows + 1 ) / 2 );
     v.elems = std::max( v.rows * v.nh, v.pairs * v.nz );
+    v.blocks = v.bd0 = 1;
     int     most = 1; // butterflies of the largest stage
     int32_t st   = v.nh;
     for ( int i = 3; i >= 0; --i )
     {
-        // logical axes at the end: d = 3 has no o0
-        const int     k = i - ( 4 - d );
-        const int64_t n = k < 0 ? 1 : L.n[k];
+        // logical axes at the end
+        const int     k = i == 3 ? d - 1 : last - ( 2 - i );
+        const int64_t n = i == 3 ? nz : ( k < first ? 1 : L.n[k] );
         vol_axis     &a = v.ax[i];
         a.n             = (int32_t)n;
-        v.sr[i]         = k < 0 ? 0 : (int32_t)L.sr[k];
-        v.sc[i]         = k < 0 ? 0 : (int32_t)L.sc[k];
+        v.sr[i]         = i < 3 && k < first ? 0 : (int32_t)L.sr[k];
+        v.sc[i]         = i < 3 && k < first ? 0 : (int32_t)L.sc[k];
         a.gs            = i < 3 ? v.sc[i] : v.sr[i];
         if ( i < 3 )
         {
@@ -1194,7 +1193,7 @@ void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std
         std::vector<any_schedule> found;
         any_schedules( n, 8, 16, any_schedule{}, found ); // every radix up to 16
         if ( found.empty() || found[0].n > VOL_MAX_STAGES )
-            return;
+            return false;
         const any_schedule *best = &found[0]; // the most even one
         for ( const any_schedule &s : found )
             if ( s.r[0] < best->r[0] )
@@ -1217,7 +1216,7 @@ void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std
         }
     }
     if ( ( 2 * v.elems + v.twelems ) * csize > vol_lds_limit() )
-        return;
+        return false;
     // forward: real axis, o2, o1, o0; backward the other way round (there the real axis's
     // first stage always builds its lines from the half spectra)
     int lo = 0, hi = 2; // first and last complex axis with stages (rows >= 2: there is one)
@@ -1234,6 +1233,23 @@ void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std
     v.mg_e1 = mulhi_magic( v.ext[1] );
     v.mg_e2 = mulhi_magic( v.ext[2] );
     v.nt    = std::min( ( most + 63 ) / 64 * 64, vol_max_threads( csize ) );
+    return true;
+}
+
+// Replace all passes by one volume pass where the array is small enough for the LDS of one
+// workgroup and for one workgroup to be faster than a launch per axis.
+void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std::vector<pass_rt> &bwd )
+{
+    const int d    = L.dim;
+    int64_t   rows = 1;
+    for ( int k = 0; k + 1 < d; ++k )
+        rows *= L.n[k];
+    const int64_t nz = L.n[d - 1];
+    pass_rt       p;
+    // one workgroup takes 7 us a direction for a few points and 12 for 4096; a launch per
+    // axis takes 13 (3D) and 17 us (4D) throughout: level at about 5500 points, 8000 in 4D
+    if ( nz < 2 || rows < 2 || rows * nz > 1536 * d || !make_tile( L, csize_of( prec ), 0, d - 2, p.vol ) )
+        return;
     p.volume = p.generic = true;
     p.N      = nz;
     p.ncols  = rows;
@@ -1245,6 +1261,65 @@ void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std
     q.inv     = true;
     fwd.assign( 1, p );
     bwd.assign( 1, q );
+}
+
+// Whether a launch of `planes` volume-pass workgroups, one per plane of the real axis (nb) and
+// its neighbour (na), beats the two passes it replaces.  Transform pairs, time of the passes
+// over the tile's, 80 shapes of 2^13..2^23 points drawn over both layouts and precisions:
+//   planes of at most 60 KB LDS: 1.02..1.34 (36 x 30 x 40 x 24 FP64 67 -> 63 us, FP32 53 -> 44,
+//     64 x 16 x 64 x 32 FP32 63 -> 55, 512 x 48 x 28 FP64 52 -> 40), but FP64 arrays of many
+//     planes or beyond 1.5 million points, where the arithmetic per value counts, 0.94..0.99,
+//     and FP32 ones beyond 6 million (2000 x 60 x 60 106 -> 108, 72^4 362 -> 492);
+//   larger planes (one or two workgroups per CU): 1.03..1.29 from 72 planes to one per CU
+//     (128 x 64 x 100 FP64 53 -> 41), 0.77..0.97 with fewer or more, and 0.96 above 136 KB.
+bool tile_faster( int64_t planes, int64_t na, int64_t nb, int csize )
+{
+    const int64_t lds = 2 * csize * std::max( na * ( nb / 2 + 1 ), ( na + 1 ) / 2 * nb );
+    if ( lds > 60 * 1024 )
+        return lds <= 136 * 1024 && planes >= 72 && planes <= 256;
+    return planes >= 24 && ( csize == 8 ? planes * na * nb <= 6 << 20 : planes <= 2304 && planes * na * nb <= 3 << 19 );
+}
+
+// Replace the real-axis pass and its neighbour's by one volume pass per plane where no plane
+// kernel exists and the plane is dense in both arrays (3D, 4D slab).
+void fuse_tiles( const ffts_layout &L, int32_t layout, int prec, std::vector<pass_rt> &fwd, std::vector<pass_rt> &bwd )
+{
+    const int d = L.dim;
+    if ( ( layout != FFTM_MI_LAYOUT_3D && layout != FFTM_MI_LAYOUT_4D_SLAB ) || (int)fwd.size() != d )
+        return; // a plane or volume pass already
+    int64_t planes = 1;
+    for ( int k = 0; k + 2 < d; ++k )
+        planes *= L.n[k];
+    const int64_t na = L.n[d - 2], nb = L.n[d - 1];
+    pass_rt       p;
+    if ( na < 2 || nb < 2 || planes > 0x7fffffff || !tile_faster( planes, na, nb, csize_of( prec ) ) ||
+         !make_tile( L, csize_of( prec ), d - 2, d - 2, p.vol ) )
+        return;
+    // 12 waves per CU in all: enough to hide latency, and no more threads per plane than that
+    // takes (3000 planes of 40 x 30 FP32 75 -> 72 us with 64 threads instead of 256)
+    vol_geom &v = p.vol;
+    v.nt        = (int32_t)std::min<int64_t>( v.nt, std::max<int64_t>( 1, ( 3072 + planes / 2 ) / planes ) * 64 );
+    v.blocks    = (int32_t)planes;
+    v.bd0       = (int32_t)L.n[d - 3];
+    for ( int i = 0; i < d - 2; ++i )
+    {
+        v.bsr[i] = L.sr[d - 3 - i];
+        v.bsc[i] = L.sc[d - 3 - i];
+    }
+    p.volume = p.generic = true;
+    p.N      = nb;
+    p.ncols  = planes * na;
+    p.kind   = KIND_R2C;
+    p.src    = BUF_IN;
+    p.dst    = BUF_OUT;
+    fwd.erase( fwd.begin() );
+    fwd.front() = p;
+    // the axis above (d >= 3: there is one) wrote what the tile reads
+    p.kind = KIND_C2R;
+    p.inv  = true;
+    bwd.pop_back();
+    p.src      = bwd[bwd.size() - 2].dst;
+    bwd.back() = p;
 }
 
 int build_ffts_passes( const ffts_layout &L, bool overwrite, std::vector<pass_rt> &fwd, std::vector<pass_rt> &bwd,
@@ -1811,6 +1886,7 @@ int fftm_mi_ffts_validate( int32_t layout, const int64_t *n, int32_t precision, 
     {
         fuse_plane( L, layout, precision, f, b );
         fuse_volume( L, precision, f, b );
+        fuse_tiles( L, layout, precision, f, b );
     }
     rc = prepare_passes( f, precision, nullptr );
     if ( rc == FFTM_MI_SUCCESS )
@@ -1859,6 +1935,7 @@ int fftm_mi_ffts_create( int32_t layout, const int64_t *n, int32_t precision, in
         {
             fuse_plane( L, layout, precision, p->fwd, p->bwd );
             fuse_volume( L, precision, p->fwd, p->bwd );
+            fuse_tiles( L, layout, precision, p->fwd, p->bwd );
         }
     }
     rc = prepare_passes( p->fwd, p->prec, &p->tb );
@@ -1990,7 +2067,7 @@ int fftm_mi_ffts_pass_bytes( fftm_mi_ffts h, int32_t backward, int32_t index, in
         return ok();
     }
     if ( p.volume )
-        *bytes = p.vol.rows * ( p.N * rs + nh * cs );
+        *bytes = p.ncols * ( p.N * rs + nh * cs );
     else if ( p.plane )
         *bytes = p.nplanes * p.NB * ( p.N * rs + nh * cs );
     else if ( p.kind == KIND_C2C )

@@ -11,9 +11,9 @@ hipError_t launch_volume_t( const vol_params<T> &p, bool fwd, hipStream_t s )
 {
     const size_t lds = sizeof( cpx<T> ) * (size_t)( 2 * p.elems + p.twelems );
     if ( fwd )
-        hipLaunchKernelGGL( ( k_volume<T, true> ), dim3( 1 ), dim3( (unsigned)p.nt ), lds, s, p );
+        hipLaunchKernelGGL( ( k_volume<T, true> ), dim3( (unsigned)p.blocks ), dim3( (unsigned)p.nt ), lds, s, p );
     else
-        hipLaunchKernelGGL( ( k_volume<T, false> ), dim3( 1 ), dim3( (unsigned)p.nt ), lds, s, p );
+        hipLaunchKernelGGL( ( k_volume<T, false> ), dim3( (unsigned)p.blocks ), dim3( (unsigned)p.nt ), lds, s, p );
     return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
-// Volume pass: a whole small transform, the real axis and every complex axis, in one
-// workgroup and one launch.
+// Volume pass: the real axis and one or more complex axes in one workgroup and one launch: a
+// whole small transform, or the planes of a larger one's two inner axes, a workgroup each.
 //
 // Problems of a few thousand points are bound by their launches: a 12 x 10 x 8 FP64 pair
 // took six kernels of 3 to 5.5 us, each nearly all latency, 28 us in all; two of these take
@@ -60,6 +60,10 @@ struct vol_geom
     int32_t  nz, nh, rows, pairs;
     int32_t  elems, twelems;   // LDS values: each of the two buffers, the twiddle tables
     int32_t  nt;               // threads
+    // workgroups: one, or one per item of up to two batch axes (extent of the faster one and
+    // the strides in the real and the complex array, faster first)
+    int32_t  blocks, bd0;
+    int64_t  bsr[2], bsc[2];
     uint32_t mg_nh, mg_e1, mg_e2;
     int32_t  sr[4], sc[4];     // element strides of the real and the complex array
 };
@@ -77,6 +81,15 @@ struct vol_kernel
 {
     using C = cpx<T>;
 
+    // the workgroup's pieces of the arrays (a kernel reads one kind and writes the other)
+    struct io
+    {
+        const C *cin;
+        C       *cout;
+        const T *rin;
+        T       *rout;
+    };
+
     __device__ static __forceinline__ int quot( int n, int d, uint32_t mg )
     {
         return d == 1 ? n : (int)__umulhi( (uint32_t)n, mg );
@@ -93,8 +106,8 @@ struct vol_kernel
     // One stage of complex axis a (gr reads HBM, gw writes HBM, sep reads the paired real lines
     // and separates them).
     template <int R>
-    __device__ static __forceinline__ void complex_stage( const vol_params<T> &p, const vol_axis &a, const vol_stage &g,
-                                                          const C *src, C *dst, const C *tw, bool sep,
+    __device__ static __forceinline__ void complex_stage( const vol_params<T> &p, const io &f, const vol_axis &a,
+                                                          const vol_stage &g, const C *src, C *dst, const C *tw, bool sep,
                                                           bool gr, bool gw )
     {
         int nbf = a.n / R, gs = a.gs;
@@ -113,7 +126,7 @@ struct vol_kernel
             C             v[R];
             if ( gr )
             {
-                const C *in = static_cast<const C *>( p.in ) + off + j * gs;
+                const C *in = f.cin + off + j * gs;
 #pragma unroll
                 for ( int r = 0; r < R; ++r )
                     v[r] = mk<T>( in[r * nbf * gs].x, in[r * nbf * gs].y );
@@ -151,7 +164,7 @@ struct vol_kernel
             dft_fixed<R, !FWD>( v );
             if ( gw )
             {
-                C *out = static_cast<C *>( p.out ) + off + d * gs;
+                C *out = f.cout + off + d * gs;
 #pragma unroll
                 for ( int m = 0; m < R; ++m )
                     out[m * ns * gs] = v[m];
@@ -169,8 +182,8 @@ struct vol_kernel
     // array (forward) or the half spectra in LDS (backward); last of the backward transform:
     // to the real array.
     template <int R>
-    __device__ static __forceinline__ void real_stage( const vol_params<T> &p, const vol_axis &a, const vol_stage &g,
-                                                       const C *src, C *dst, const C *tw, bool first,
+    __device__ static __forceinline__ void real_stage( const vol_params<T> &p, const io &f, const vol_axis &a,
+                                                       const vol_stage &g, const C *src, C *dst, const C *tw, bool first,
                                                        bool last )
     {
         int nbf = a.n / R, gs = a.gs;
@@ -183,8 +196,8 @@ struct vol_kernel
             C          v[R];
             if ( first && FWD )
             {
-                const T *sa = static_cast<const T *>( p.in ) + row_offset( p, 2 * q, p.sr ) + j * gs;
-                const T *sb = vb ? static_cast<const T *>( p.in ) + row_offset( p, 2 * q + 1, p.sr ) + j * gs : sa;
+                const T *sa = f.rin + row_offset( p, 2 * q, p.sr ) + j * gs;
+                const T *sb = vb ? f.rin + row_offset( p, 2 * q + 1, p.sr ) + j * gs : sa;
 #pragma unroll
                 for ( int r = 0; r < R; ++r )
                     v[r] = mk<T>( sa[r * nbf * gs], sb[r * nbf * gs] );
@@ -238,13 +251,13 @@ struct vol_kernel
             dft_fixed<R, !FWD>( v );
             if ( last && !FWD )
             {
-                T *da = static_cast<T *>( p.out ) + row_offset( p, 2 * q, p.sr ) + d * gs;
+                T *da = f.rout + row_offset( p, 2 * q, p.sr ) + d * gs;
 #pragma unroll
                 for ( int m = 0; m < R; ++m )
                     da[m * ns * gs] = v[m].x;
                 if ( vb )
                 {
-                    T *db = static_cast<T *>( p.out ) + row_offset( p, 2 * q + 1, p.sr ) + d * gs;
+                    T *db = f.rout + row_offset( p, 2 * q + 1, p.sr ) + d * gs;
 #pragma unroll
                     for ( int m = 0; m < R; ++m )
                         db[m * ns * gs] = v[m].y;
@@ -260,25 +273,30 @@ struct vol_kernel
     }
 
     template <int R>
-    __device__ static __forceinline__ void stage( const vol_params<T> &p, const vol_axis &a, bool real,
+    __device__ static __forceinline__ void stage( const vol_params<T> &p, const io &f, const vol_axis &a, bool real,
                                                   const vol_stage &g, const C *src, C *dst, const C *tw, bool sep,
                                                   bool gr, bool gw )
     {
         // the markers keep the radices' register arrays apart, see any_kernel::stage_r
         if ( real )
         {
-            real_stage<R>( p, a, g, src, dst, tw, gr, gw );
+            real_stage<R>( p, f, a, g, src, dst, tw, gr, gw );
             asm volatile( "; radix %0 real" ::"n"( R ) );
         }
         else
         {
-            complex_stage<R>( p, a, g, src, dst, tw, sep, gr, gw );
+            complex_stage<R>( p, f, a, g, src, dst, tw, sep, gr, gw );
             asm volatile( "; radix %0" ::"n"( R ) );
         }
     }
 
     __device__ static __forceinline__ void run( const vol_params<T> &p, C *lds )
     {
+        const int     item = p.blocks > 1 ? (int)ordered_tile( 0 ) : 0;
+        const int     b1 = item / p.bd0, b0 = item - b1 * p.bd0;
+        const int64_t oc = b0 * p.bsc[0] + b1 * p.bsc[1], orl = b0 * p.bsr[0] + b1 * p.bsr[1];
+        const io      f{ static_cast<const C *>( p.in ) + oc, static_cast<C *>( p.out ) + oc,
+                         static_cast<const T *>( p.in ) + orl, static_cast<T *>( p.out ) + orl };
         C  *src = lds, *dst = lds + p.elems;
         C  *tw  = lds + 2 * p.elems;
         // the twiddle tables of the axes with more than one stage
@@ -320,21 +338,21 @@ struct vol_kernel
                 const C *twl = tw + a.tw;
                 switch ( r )
                 {
-                case 2: stage<2>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 3: stage<3>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 4: stage<4>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 5: stage<5>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 6: stage<6>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 7: stage<7>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 8: stage<8>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 9: stage<9>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 10: stage<10>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 11: stage<11>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 12: stage<12>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 13: stage<13>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 14: stage<14>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 15: stage<15>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
-                case 16: stage<16>( p, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 2: stage<2>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 3: stage<3>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 4: stage<4>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 5: stage<5>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 6: stage<6>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 7: stage<7>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 8: stage<8>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 9: stage<9>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 10: stage<10>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 11: stage<11>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 12: stage<12>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 13: stage<13>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 14: stage<14>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 15: stage<15>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
+                case 16: stage<16>( p, f, a, real, g, src, dst, twl, sep, gr, gw ); break;
                 default: break; // the host plans no other radix
                 }
                 __syncthreads();
