@@ -203,7 +203,7 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
                 continue;
             std::rotate( s.r, s.r + f, s.r + f + 1 );
             // column-fastest tiles: a power of two of columns; line-fastest: any number of lines
-            for ( int64_t c = 1; c <= 64; c += loadb ? c : std::max<int64_t>( 1, c / 6 ) )
+            for ( int64_t c = 1; c <= ANY_MAX_COLS; c += loadb ? c : std::max<int64_t>( 1, c / 6 ) )
             {
                 if ( c > 1 && line * c * csize > ( loadb ? 81920 : 45056 ) )
                     break;
@@ -253,28 +253,54 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
     return true;
 }
 
-// Compiled 3/5/7-smooth lengths whose contiguous lines the runtime-length kernel transforms
-// faster, with both measured at 2^22 / 2^26 values (time of the compiled one over its time):
-//   R2C FP32 to 288 points, FP64 to 80: 1.04..2.9 / 1.0..2.9 (the compiled tiles hold few
-//   values per thread there and read 4-byte reals), 0.84..1.2 beyond;
-//   C2C FP32 to 56, FP64 to 144: 0.94..1.7 / 0.97..1.5, beyond that down to 0.7;
-//   FP32 from 1000 points where radices up to 16 save a stage and the odd part is above 15
-//   (1000 = 10 10 10 instead of 8 5 5 5): 1.0..1.5 / 1.0..1.4; 0.8..1.1 for 2^k 3, 5, 9 or 15.
-// C2R lines, and columns, which differ by less and in both directions, stay compiled.
-bool runtime_rows( const pass_rt &p, int csize )
+// Compiled 3/5/7-smooth lengths that the runtime-length kernel transforms faster.  Measured:
+// both kernels on all of them at 2^16, 2^19, 2^22 and 2^24 values, rows also at 2^26; the
+// ranges are the compiled kernel's time over the runtime one's.
+//   FP32 columns from 224 points: 0.94..1.8, 1.2 on average (1920 1.34 1.29 1.28 1.14; the
+//     compiled tiles are of one size, and 1000 = 10 10 10 instead of 8 5 5 5 saves a stage);
+//   FP32 R2C rows to 288 points 1.0..3.2 (the compiled tiles hold few values per thread there
+//     and read 4-byte reals), to 480 0.96..1.2, to 1152 1.0..1.4 up to 2^23 values;
+//   FP32 C2C rows from 24 to 56 points 1.0..1.7, to 480 0.93..1.5 where the odd part is above 5
+//     or the power of two below 32, 12 points 1.3 from 2^20 values (0.9 below);
+//   FP32 C2R rows of 8 times an odd number to 120 points 0.97..1.7, 2^k 7 and 2^k 9 from 112 to
+//     480 points 0.94..1.3;
+//   FP32 rows from 1000 points where radices up to 16 save a stage and the odd part is above 15:
+//     0.95..2.0; 0.8..1.1 for 2^k 3, 5, 9 or 15;
+//   FP64 rows where the compiled schedule starts with radix 4 or 16 (a power of two of 4, 16 or
+//     128): C2R to 480 points 0.93..3.2, R2C 0.96..1.8, C2C 0.92..1.8; the others 0.7..1.1 but for
+//     R2C to 80 points (0.94..1.3) and four-stage C2R lines (288, 480: 1.1..2.3).
+// FP64 columns (0.6..1.2), and what lies beyond 2^24 values where that was not measured, stay.
+bool runtime_faster( const pass_rt &p, int csize )
 {
-    if ( p.loadb || pow2_length( p.N ) || p.kind == KIND_C2R )
+    if ( pow2_length( p.N ) || ( p.loadb && ( p.kind != KIND_C2C || csize != 8 ) ) )
         return false;
-    if ( p.N <= ( p.kind == KIND_R2C ? ( csize == 8 ? 288 : 80 ) : ( csize == 8 ? 56 : 144 ) ) )
-        return true;
-    if ( csize != 8 || p.N < 1000 )
-        return false;
-    int64_t odd = p.N;
-    while ( odd % 2 == 0 )
-        odd /= 2;
-    std::vector<any_schedule> found;
-    any_schedules( p.N, csize, 16, any_schedule{}, found );
-    return odd > 15 && !found.empty() && found[0].n < make_rplan( (int)p.N ).n;
+    const int64_t N = p.N, two = N & -N, odd = N / two, values = p.ncols * N;
+    const bool    within = values <= (int64_t)1 << 24;
+    if ( p.loadb )
+        return within && N >= 224;
+    if ( csize != 8 )
+    {
+        if ( p.kind == KIND_R2C && N <= 80 )
+            return true;
+        const bool lead = two == 4 || two == 16 || two == 128;
+        return N <= 480 && ( N <= 144 || within ) &&
+               ( lead || ( p.kind == KIND_C2R && make_rplan( (int)N ).n >= 4 ) );
+    }
+    if ( N >= 1000 && odd > 15 )
+    {
+        std::vector<any_schedule> found;
+        any_schedules( N, csize, 16, any_schedule{}, found );
+        if ( !found.empty() && found[0].n < make_rplan( (int)N ).n )
+            return true;
+    }
+    switch ( p.kind )
+    {
+    case KIND_R2C: return N <= 288 || ( N <= 480 && within ) || ( N <= 1152 && values <= 1 << 23 );
+    case KIND_C2R: return within && ( ( two == 8 && N <= 120 ) || ( two >= 16 && N <= 480 && ( odd == 7 || odd == 9 ) ) );
+    default:
+        return N < 24 ? N == 12 && values >= 1 << 20
+                      : N <= 56 || ( N <= 480 && within && ( odd > 5 || two < 32 ) );
+    }
 }
 
 // Decide how a pass of length N runs (fixed kernel or generic); fills N-dependent fields.
@@ -282,7 +308,7 @@ bool runtime_rows( const pass_rt &p, int csize )
 int configure_kernel( pass_rt &p, int prec, bool plan )
 {
     if ( fixed_supported( p.N ) &&
-         !( plan && runtime_rows( p, csize_of( prec ) ) &&
+         !( plan && runtime_faster( p, csize_of( prec ) ) &&
             make_any_plan( p.N, csize_of( prec ), p.loadb, p.kind, p.ncols, p.any ) ) )
     {
         p.generic = false;
@@ -619,11 +645,13 @@ int default_order( const pass_rt &p )
 //     200, FP64 414 -> 400, 414 -> 411;
 //   columns, N >= 1024 (a 128-byte row segment of them is 128 KB and more): split exchange
 //     with full row segments (3): 1024 x 1024 x 256 FP32 x 943 -> 534, y 496 -> 454, FP64
-//     1024 x 512 x 256 885 -> 577; FP32 arrays that the cache holds are 2-15 % better off
-//     with 2 (1024 x 128 x 128 31.9 -> 29.0 against 34.0) up to N = 2048;
+//     1024 x 512 x 256 885 -> 577; arrays that the cache holds are 2-15 % better off with 2
+//     (FP32 1024 x 128 x 128 31.9 -> 29.0 against 34.0; FP64 1024 x 129 6.0 against 8.7), from
+//     2048 points on only below 32 MB (FP32 2048 columns of 2048 points 19.1 -> 17.8, 512 of them
+//     10.4 against 14.4; FP64 4096 points 27.3 -> 23.6 at 512 columns, 18.6 level at 256);
 //   columns, N = 256: 3 beyond the cache (256 x 1024 x 512 FP32 221 -> 193, 256^3 FP64 49.0
 //     -> 46.8), level with 0 and 2 within it for FP32 and 13 % slower;
-//   columns, N = 128, FP64: split exchange (6), 64 x 128 x 1024 26.2 -> 24.1;
+//   columns, N = 128, FP64: split exchange (6), 64 x 128 x 1024 26.2 -> 24.1, level below 32 MB;
 //   FP32 real rows, N = 64 and 256: 2 (R2C 12.6 -> 11.5, 27.0 -> 26.3; C2R 13.6 -> 12.3, 27.4
 //     -> 26.2), N = 128 R2C: 6 within the cache (27.7 -> 25.6), 5 beyond it (431 -> 403);
 //   FP16-stored columns: 6 where FP16 lines are read (512^3 157 -> 141, 197 -> 188, 177 ->
@@ -653,9 +681,12 @@ int default_shape( const pass_rt &p, int csize )
     }
     if ( !p.loadb )
         return 0;
-    if ( csize == 8 )
-        return p.N < 256 ? 0 : ( p.N == 256 ? ( beyond ? 3 : 2 ) : ( p.N >= 4096 || ( p.N >= 1024 && beyond ) ? 3 : 2 ) );
-    return p.N >= 1024 ? 3 : ( p.N == 512 ? 2 : ( p.N == 256 ? ( beyond ? 3 : 0 ) : ( p.N == 128 ? 6 : 0 ) ) );
+    const bool wide = p.N >= 2048 ? bytes >= 32 << 20 : beyond;
+    if ( p.N >= 512 )
+        return p.N >= 1024 && wide ? 3 : 2;
+    if ( p.N == 256 )
+        return beyond ? 3 : ( csize == 8 ? 2 : 0 );
+    return csize == 16 && p.N == 128 && bytes >= 32 << 20 ? 6 : 0;
 }
 
 // Default tile shape of the fused filter pass (shapes 0, 2, 4): twice the threads per
@@ -1271,12 +1302,13 @@ void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std
 //     planes or beyond 1.5 million points, where the arithmetic per value counts, 0.94..0.99,
 //     and FP32 ones beyond 6 million (2000 x 60 x 60 106 -> 108, 72^4 362 -> 492);
 //   larger planes (one or two workgroups per CU): 1.03..1.29 from 72 planes to one per CU
-//     (128 x 64 x 100 FP64 53 -> 41), 0.77..0.97 with fewer or more, and 0.96 above 136 KB.
+//     (128 x 64 x 100 FP64 53 -> 41), 0.77..0.97 with fewer or more, and 0.96 above 136 KB; 0.90
+//     where the real rows are powers of two (128 x 64 x 128 FP64 45.5 -> 50).
 bool tile_faster( int64_t planes, int64_t na, int64_t nb, int csize )
 {
     const int64_t lds = 2 * csize * std::max( na * ( nb / 2 + 1 ), ( na + 1 ) / 2 * nb );
     if ( lds > 60 * 1024 )
-        return lds <= 136 * 1024 && planes >= 72 && planes <= 256;
+        return lds <= 136 * 1024 && planes >= 72 && planes <= 256 && !pow2_length( nb );
     return planes >= 24 && ( csize == 8 ? planes * na * nb <= 6 << 20 : planes <= 2304 && planes * na * nb <= 3 << 19 );
 }
 

@@ -9,11 +9,11 @@ import pytest
 
 from helpers import check_close, from_gpu, to_gpu
 
-# compiled lengths whose rows take the runtime kernel (12, 20, 48, 56, 100, 144, 1000, 1680)
-# and others; 1..15: single stages; 3125 = 5^5 five stages; primes 11 and 13 alone, squared and cubed;
+# compiled lengths that take the runtime kernel in some kind, direction or precision (12, 20, 24,
+# 48, 56, 72, 100, 120, 144, 224, 240, 288, 400, 480, 576, 1000, 1152, 1680, 1920) and others; 1..15: single stages; 3125 = 5^5 five stages; primes 11 and 13 alone, squared and cubed;
 # the largest lengths each precision takes
-LENGTHS = [1, 3, 6, 7, 9, 11, 12, 13, 14, 15, 18, 20, 22, 26, 39, 45, 48, 56, 99, 100, 125, 143, 144, 169, 175, 234, 250, 330, 343, 420, 625, 720,
-           1000, 1001, 1080, 1331, 1680, 2016, 2197, 3125, 3993, 4004, 4095]
+LENGTHS = [1, 3, 6, 7, 9, 11, 12, 13, 14, 15, 18, 20, 22, 24, 26, 39, 45, 48, 56, 72, 99, 100, 120, 125, 143, 144, 169, 175,
+           224, 234, 240, 250, 288, 330, 343, 400, 420, 480, 576, 625, 720, 1000, 1001, 1080, 1152, 1331, 1680, 1920, 2016, 2197, 3125, 3993, 4004, 4095]
 MAX_LENGTH = {"float32": 4096, "float64": 2048}
 
 
