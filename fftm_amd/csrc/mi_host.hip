@@ -1112,7 +1112,7 @@ int plane_partner( int32_t layout )
 }
 
 // Replace the real-axis pass and the C2C pass along `B` by one plane pass when the
-// (B x A) half-spectrum plane fits in LDS and there are at least 64 planes.
+// (B x A) half-spectrum plane fits in LDS.
 void fuse_plane( const ffts_layout &L, int32_t layout, int prec, std::vector<pass_rt> &fwd, std::vector<pass_rt> &bwd )
 {
     const int     d  = L.dim;
@@ -1129,10 +1129,12 @@ void fuse_plane( const ffts_layout &L, int32_t layout, int prec, std::vector<pas
             nplanes *= L.n[k];
             other[no++] = k;
         }
-    // Fewer planes than CUs still pay off: the fused pair has four passes instead of six,
-    // and problems this small are bound by their launches (128^3 FP64 round trip 62 ->
-    // 50 us, 64^3 30 -> 24 us).  Below 64 planes the split passes keep more workgroups.
-    if ( nplanes < 64 )
+    // Fewer planes than CUs still pay off: a launch less in each direction, and a plane's time is
+    // its chain of latencies however many there are (pairs, passes -> plane: 8 planes of 64^2
+    // FP32 22.4 -> 15.4 us, 32 of them FP64 25.1 -> 19.3, 8 of 128^2 FP32 27.1 -> 23.3; 128^3 FP64
+    // 62 -> 49).  FP64 planes of 128^2 take 12 us at the least: 32 of them 37.5 -> 38.7, 48
+    // 44.7 -> 42.8.
+    if ( prec != FFTM_MI_F32 && na >= 128 && nplanes < 48 )
         return;
     pass_rt p;
     p.plane   = true;

@@ -26,10 +26,10 @@ hipError_t launch_plane_n( const plane_params<T> &p, bool fwd, hipStream_t s )
     return hipGetLastError();
 }
 
-template <typename T, int N>
+template <typename T, int N, bool WIDE>
 hipError_t launch_plane_rx_n( const plane_params<T> &p, bool fwd, hipStream_t s )
 {
-    using G = plane_rx_geom<N, (int)sizeof( cpx<T> )>;
+    using G = plane_rx_geom<N, (int)sizeof( cpx<T> ), WIDE>;
     if ( p.nplanes <= 0 )
         return hipSuccess;
     const int64_t groups = ( p.nplanes + G::PPW - 1 ) / G::PPW;
@@ -39,25 +39,26 @@ hipError_t launch_plane_rx_n( const plane_params<T> &p, bool fwd, hipStream_t s 
     // real rows staged through LDS unless B is contiguous in the real array
     const bool staged = p.rb != 1;
     if ( fwd && staged )
-        hipLaunchKernelGGL( ( k_plane_rx<T, N, true, true> ), grid, block, 0, s, p );
+        hipLaunchKernelGGL( ( k_plane_rx<T, N, true, true, WIDE> ), grid, block, 0, s, p );
     else if ( fwd )
-        hipLaunchKernelGGL( ( k_plane_rx<T, N, true, false> ), grid, block, 0, s, p );
+        hipLaunchKernelGGL( ( k_plane_rx<T, N, true, false, WIDE> ), grid, block, 0, s, p );
     else if ( staged )
-        hipLaunchKernelGGL( ( k_plane_rx<T, N, false, true> ), grid, block, 0, s, p );
+        hipLaunchKernelGGL( ( k_plane_rx<T, N, false, true, WIDE> ), grid, block, 0, s, p );
     else
-        hipLaunchKernelGGL( ( k_plane_rx<T, N, false, false> ), grid, block, 0, s, p );
+        hipLaunchKernelGGL( ( k_plane_rx<T, N, false, false, WIDE> ), grid, block, 0, s, p );
     return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_plane_rx_t( const plane_params<T> &p, int n, bool fwd, hipStream_t s )
 {
+    const bool wide = plane_rx_wide( n, (int)sizeof( cpx<T> ), p.nplanes );
     switch ( n )
     {
-    case 16: return launch_plane_rx_n<T, 16>( p, fwd, s );
-    case 32: return launch_plane_rx_n<T, 32>( p, fwd, s );
-    case 64: return launch_plane_rx_n<T, 64>( p, fwd, s );
-    case 128: return launch_plane_rx_n<T, 128>( p, fwd, s );
+    case 16: return launch_plane_rx_n<T, 16, false>( p, fwd, s );
+    case 32: return wide ? launch_plane_rx_n<T, 32, true>( p, fwd, s ) : launch_plane_rx_n<T, 32, false>( p, fwd, s );
+    case 64: return wide ? launch_plane_rx_n<T, 64, true>( p, fwd, s ) : launch_plane_rx_n<T, 64, false>( p, fwd, s );
+    case 128: return wide ? launch_plane_rx_n<T, 128, true>( p, fwd, s ) : launch_plane_rx_n<T, 128, false>( p, fwd, s );
     default: return hipErrorInvalidValue;
     }
 }

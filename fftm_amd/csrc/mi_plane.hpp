@@ -367,7 +367,7 @@ __global__ void __launch_bounds__( ( plane_geom<NA, NB, (int)sizeof( cpx<T> ), P
 // k_plane's, so the two kernels give bitwise equal results and the tuner can choose
 // either.
 // ---------------------------------------------------------------------------
-template <int N, int CS>
+template <int N, int CS, bool WIDE>
 struct plane_rx_geom
 {
     static constexpr int NAH = N / 2 + 1;
@@ -376,7 +376,8 @@ struct plane_rx_geom
     // workgroup (smaller LDS tiles) keep more workgroups in flight per CU: at 64 points,
     // one plane per workgroup runs the 64^4 plane passes 13-15 % faster than two
     static constexpr int PPW = N <= 16 ? 8 : ( N <= 32 ? 2 : 1 );
-    static constexpr int NT  = N >= 128 ? 512 : 256;
+    // threads: half a butterfly set each (WIDE) where few planes leave the chip to latency
+    static constexpr int NT  = ( N >= 128 ? 512 : 256 ) * ( WIDE ? 2 : 1 );
     static constexpr int XSH = 3;                    // one pad element every 8
     static constexpr int PX  = N + ( N >> XSH ) + 1; // row lines (A axis): odd pitch
     // column lines (B axis): an even pitch when consecutive threads take the butterflies
@@ -389,6 +390,20 @@ struct plane_rx_geom
     static constexpr int TOTAL = ELEMS + 2 * N; // + twiddle tables (A, then B)
     static constexpr int BYTES = TOTAL * CS;
 };
+
+// WIDE or not, by the number of planes.  Microseconds forward / inverse, without -> with:
+//   128 points, 128 planes: FP32 10.0 / 11.5 -> 9.2 / 10.1, FP64 14.5 / 15.9 -> 13.9 / 14.7;
+//   512 planes: FP32 17.7 / 19.8 -> 17.1 / 22.6, FP64 (one workgroup per CU either way)
+//   36.0 / 38.2 -> 34.7 / 37.2;
+//   64 points, 64 planes: FP32 5.6 / 6.0 -> 4.6 / 4.9, FP64 6.6 / 7.1 -> 5.6 / 6.0; 1024 planes:
+//   10.0 / 11.1 -> 9.8 / 10.4, 15.6 / 17.3 -> 15.0 / 17.9; 4096: 25.6 / 29.1 -> 26.8 / 28.7;
+//   32 points, 1024 planes: 5.1 / 5.8 -> 5.1 / 5.3, 6.8 / 7.0 -> 6.4 / 6.6; 4096: 10.5 / 11.3 ->
+//   11.8 / 12.0.
+// The 64-point planes of a 64^4 pencil (4096) take 149 us a pair without, 155 with.
+inline bool plane_rx_wide( int n, int csize, int64_t nplanes )
+{
+    return n >= 128 ? csize == 16 || nplanes <= 256 : nplanes <= 1024;
+}
 
 // Stockham stages of NL lines of length N: stage 0 reads ld(line, e), the last stage
 // calls st(line, e, value), and stages in between exchange through LDS at
@@ -489,12 +504,12 @@ struct rx_lines
 // array): the real rows go through LDS with consecutive threads along A.  Otherwise the
 // threads walk the rows q, and p.pair (set by the host for rb = 1, even real-array
 // offsets and an aligned real array) moves rows 2q, 2q+1 as one pair of values.
-template <typename T, int N, bool FWD, bool STAGED>
-__global__ void __launch_bounds__( ( plane_rx_geom<N, (int)sizeof( cpx<T> )>::NT ) )
+template <typename T, int N, bool FWD, bool STAGED, bool WIDE>
+__global__ void __launch_bounds__( ( plane_rx_geom<N, (int)sizeof( cpx<T> ), WIDE>::NT ) )
     k_plane_rx( const plane_params<T> p )
 {
     using C               = cpx<T>;
-    using G               = plane_rx_geom<N, (int)sizeof( C )>;
+    using G               = plane_rx_geom<N, (int)sizeof( C ), WIDE>;
     using V2              = typename pair_of<T>::type;
     constexpr int NT      = G::NT;
     constexpr int PPW     = G::PPW;
