@@ -207,6 +207,10 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
             {
                 if ( c > 1 && line * c * csize > ( loadb ? 81920 : 45056 ) )
                     break;
+                // an array of few tiles is bound by one tile's chain of latencies: no larger
+                // ones than fill a 64-byte row or a wave where that leaves under 128 of them
+                if ( c > ( loadb ? 64 / csize : ( 320 + N - 1 ) / N ) && ( lines + c - 1 ) / c < 128 )
+                    break;
                 // threads that hold about 5 to 16 values each
                 const int64_t v0 = N * c / 16, v1 = N * c / 5;
                 for ( int nt = (int)std::max<int64_t>( 64, v0 / 64 * 64 );
