@@ -139,13 +139,10 @@ uint32_t mulhi_magic( int64_t d )
 // is better; negative if a stage needs more butterflies per thread than the kernel holds.
 // The terms: lanes idle in some stage (1: none), wavefronts per CU short of 24, octaves off
 // 256 threads, bank conflicts of stage 0's writes (stride r0), bytes in flight per CU short
-// of 128 KB, loads per thread in stage 0, trips per stage, LDS, short rows, values held per
-// thread, a last round of workgroups that is nearly empty.  The weights were fitted to 30 000
-// measured (schedule, cols, nt) of 31 lengths 12..2000 in all kinds, 2^22 and 2^25 values: the
-// choice takes 1.03..1.05 times the best measured time there, the fixed-size tiles before it
-// 1.07..1.14.  Those of FP64 rows come from 25 000 more of 12 lengths 36..400: 1.025, 1.041
-// before (gradient of 192 x 160 x 144 237 -> 232 us); the same for FP32 rows gained 3 % on
-// 1000 points and lost 1 % on 330, and was left out.
+// of 128 KB, loads per thread in stage 0, trips per stage, LDS, short rows.  The weights were
+// fitted to 30 000 measured (schedule, cols, nt) of 31 lengths 12..2000 in all kinds, 2^22
+// and 2^25 values: the choice takes 1.03..1.05 times the best measured time there, the
+// fixed-size tiles before it 1.07..1.14.
 double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool loadb, int64_t cols, int nt,
                  int64_t lines )
 {
@@ -168,15 +165,12 @@ double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool
     const double conflict = std::max( 0, ( s.r[0] & -s.r[0] ) - 2 );
     const double row      = std::max( 0.0, 1.0 - cols * csize / 128.0 );
     const double sector   = loadb && cols * csize < 32 ? 10 : 0; // below one only where nothing else fits
-    const double tiles    = (double)( ( lines + cols - 1 ) / cols );
-    const double fill     = std::max( 0.0, 2.0 - 2.0 * tiles / 512.0 );
-    const double held     = (double)( N * cols ) / nt / 16.0;
-    const double rounds   = tiles / ( 256.0 * wgs );
-    const double tail     = std::min( 1.0, std::ceil( rounds ) / rounds - 1.0 );
+    const double fill     = std::max( 0.0, 2.0 - 2.0 * (double)( ( lines + cols - 1 ) / cols ) / 512.0 );
     if ( csize == 8 )
         return loadb ? 1 + sector + fill + 0.8 * slots + 0.8 * waves + 0.1 * octaves + 0.05 * conflict + 0.3 * inflight -
                            0.8 * first + 0.8 * row
-                     : 1 + fill + 0.5 * slots + 0.8 * waves + 0.03 * octaves + 0.45 * lds / 65536 - 0.3 * held + 0.1 * tail;
+                     : 1 + fill + 0.8 * slots + 0.8 * waves + 0.1 * octaves + 0.05 * conflict - 0.1 * first + 0.1 * lds / 65536 +
+                           0.1 / 16 * ( (double)( N * cols ) / nt );
     return loadb ? 1 + sector + fill + 0.8 * slots + 0.5 * octaves + 0.3 * conflict + 0.8 * inflight - 0.3 * first +
                        0.8 * lds / 65536
                  : 1 + fill + 0.5 * slots + 0.3 * octaves + 0.05 * conflict - 0.1 * first + 0.3 * trips + 0.8 * lds / 65536;
