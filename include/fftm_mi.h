@@ -195,7 +195,7 @@ int fftm_mi_ffts_run_pass( fftm_mi_ffts h, int32_t backward, int32_t index, cons
  * FP16-storage passes (FFTM_MI_F32_H16) have shapes 0, 2, 6 and 7, hi + lo storage passes
  * (FFTM_MI_F32_H16X2) shapes 0, 2 and 6.  Lengths compiled
  * with the default shape only (below 64, and the 3/5/7-smooth lengths) run the default
- * shape whatever the variant; plane and any-radix passes also keep their own tile order. */
+ * shape whatever the variant, as runtime-length passes do; volume passes have one of each. */
 int fftm_mi_ffts_set_pass_variant( fftm_mi_ffts h, int32_t backward, int32_t index, int32_t variant );
 int fftm_mi_ffts_get_pass_variant( fftm_mi_ffts h, int32_t backward, int32_t index, int32_t *variant );
 /* Algorithmic HBM bytes one pass moves (reads + writes of its input and output). */
