@@ -2541,16 +2541,25 @@ std::string problem_key( const fftm_mi_ffts_s &h )
     if ( h.layout != FFTM_MI_LAYOUT_3D )
         o << "x" << h.n[3];
     o << ( h.h16x2 ? "_F32_H16X2" : ( h.h16 ? "_F32_H16" : ( h.prec == FFTM_MI_F32 ? "_F32" : "_F64" ) ) );
-    // creation flags change the pass list (plane fusion, in-place backward): records are
-    // per pass index, so a handle only takes records measured with the same flags
+    // records are per pass index, so a handle only takes records measured on the same pass
+    // list: creation flags change it (plane fusion, in-place backward), and so do the fusions
+    // that a problem of this size takes.  Keys without a suffix are those of one pass per axis
+    // and of plane passes over 64 planes and more; caches that hold them stay valid.
     if ( h.flags )
         o << "_FLAGS" << h.flags;
+    const pass_rt &first = h.fwd.front();
+    if ( first.volume )
+        o << ( h.fwd.size() == 1 ? "_VOLUME" : "_TILES" );
+    else if ( first.plane && first.nplanes < 64 )
+        o << "_PLANES";
     return o.str();
 }
 
-std::string pass_key( const std::string &prob, int bw, size_t i )
+// Runtime-length passes have keys of their own: a record of the compiled kernel of that length
+// (or of one with a fixed tile order) says nothing about them.
+std::string pass_key( const std::string &prob, int bw, size_t i, const pass_rt &p )
 {
-    return prob + ( bw ? "_BWD" : "_FWD" ) + std::to_string( i );
+    return prob + ( bw ? "_BWD" : "_FWD" ) + std::to_string( i ) + ( p.generic && !p.volume ? "_RUNTIME" : "" );
 }
 
 __global__ void k_count_diff( const uint32_t *a, const uint32_t *b, int64_t n, unsigned long long *count )
@@ -2790,7 +2799,7 @@ int fftm_mi_ffts_load_tuning( fftm_mi_ffts h, const char *cache_path, int32_t *a
         std::vector<pass_rt> &v = bw ? h->bwd : h->fwd;
         for ( size_t i = 0; i < v.size(); ++i )
         {
-            auto it = m.find( pass_key( prob, bw, i ) );
+            auto it = m.find( pass_key( prob, bw, i, v[i] ) );
             if ( it == m.end() )
                 continue;
             const int var = std::atoi( it->second.c_str() );
@@ -2971,7 +2980,7 @@ int fftm_mi_ffts_autotune( fftm_mi_ffts h, const void *real_in, void *spectrum_o
                 const double med = ms.size() % 2 ? ms[ms.size() / 2] : 0.5 * ( ms[ms.size() / 2 - 1] + ms[ms.size() / 2] );
                 char         pfx[32];
                 std::snprintf( pfx, sizeof( pfx ), "_CANDIDATE_%03d_", var );
-                const std::string k = pass_key( prob, bw, i ) + pfx;
+                const std::string k = pass_key( prob, bw, i, cur ) + pfx;
                 std::ostringstream mo;
                 mo << std::setprecision( 9 ) << med;
                 rec[k + "VALID"]     = valid ? "1" : "0";
@@ -2986,10 +2995,10 @@ int fftm_mi_ffts_autotune( fftm_mi_ffts h, const void *real_in, void *spectrum_o
             {
                 h->flt_ready                    = false;
                 v[i].var                        = best;
-                rec[pass_key( prob, bw, i )]    = std::to_string( best );
+                rec[pass_key( prob, bw, i, cur )] = std::to_string( best );
                 std::ostringstream mo;
                 mo << std::setprecision( 9 ) << best_ms;
-                rec[pass_key( prob, bw, i ) + "_WINNER_MEDIAN_MS"] = mo.str();
+                rec[pass_key( prob, bw, i, cur ) + "_WINNER_MEDIAN_MS"] = mo.str();
             }
         }
     }
