@@ -1594,7 +1594,7 @@ void launch_shell_gradient_t( fftm_mi_ffts_s *h, const void *grad_spectrum, cons
 {
     unsigned        blocks = 0;
     const spec_walk w      = make_walk( h->sg, 512, SHELL_BLOCKS, blocks );
-    const size_t    lds    = sizeof( double ) * (size_t)nshells + sizeof( int ) * (size_t)( nshells + 1 );
+    const size_t    lds    = sizeof( double ) * (size_t)nshells;
     hipLaunchKernelGGL( k_shell_partials<T>, dim3( blocks ), dim3( 512 ), lds, h->stream, w, nshells, h->sg.kmax2,
                         static_cast<const cpx<T> *>( grad_spectrum ), static_cast<const cpx<T> *>( spectrum ), partials );
     hipLaunchKernelGGL( k_shell_reduce<T>, dim3( ( nshells + 3 ) / 4 ), dim3( 256 ), 0, h->stream, partials,

@@ -124,49 +124,27 @@ __global__ void __launch_bounds__( 256 ) k_filter_multiply( int64_t total, const
     }
 }
 
-// Lower bounds of the radial shells in |k|^2, in LDS: shell s holds thr[s] <= |k|^2 <
-// thr[s + 1], i.e. the largest s with s^2 kmax2 <= S^2 |k|^2 (see shell_of; all integers);
-// the last shell is open.
-__device__ __forceinline__ void shell_bounds( int *thr, int S, int64_t kmax2 )
-{
-    const int64_t d = (int64_t)S * S;
-    for ( int s = threadIdx.x; s <= S; s += blockDim.x )
-        thr[s] = s == S ? 0x7fffffff : (int)( ( (int64_t)s * s * kmax2 + d - 1 ) / d );
-    __syncthreads();
-}
-
-// shell of k2, walking from shell s (a walk's neighbouring bins lie in neighbouring shells)
-__device__ __forceinline__ int shell_from( const int *thr, int s, int k2 )
-{
-    while ( k2 >= thr[s + 1] )
-        ++s;
-    while ( k2 < thr[s] )
-        --s;
-    return s;
-}
-
-// out[i] = coeffs[shell(i)] in[i]
+// out[i] = coeffs[shell(i)] in[i].  A thread's next bin lies w.rows rows on and so, in a large
+// array, many shells away: walking a table of shell bounds from the last bin's shell cost a
+// dependent LDS read per shell passed (128^3 FP32: 6.8 us with 32 shells, 9.5 with 100, 51 with
+// 1024; 5.5 with any number now, 256^3 27.0 -> 21.7 with 32).
 template <typename T>
 __global__ void __launch_bounds__( 256 )
     k_shell_multiply( const spec_walk w, int S, int64_t kmax2, const cpx<T> *in, cpx<T> *out, const T *coeffs )
 {
-    __shared__ int thr[MAX_SHELLS + 1];
-    shell_bounds( thr, S, kmax2 );
-    int s = -1;
     walk_rows( w, [&]( const int64_t( &o )[4], const int( &k2 )[4], const int( & )[4] ) {
         cpx<T> z[4];
+        T      h[4];
 #pragma unroll
         for ( int u = 0; u < 4; ++u )
+        {
             z[u] = in[o[u] < w.total ? o[u] : o[0]];
-        if ( s < 0 )
-            s = shell_of( k2[0], S, kmax2 );
+            h[u] = coeffs[shell_of( k2[u], S, kmax2 )];
+        }
 #pragma unroll
         for ( int u = 0; u < 4; ++u )
             if ( o[u] < w.total )
-            {
-                s         = shell_from( thr, s, k2[u] );
-                out[o[u]] = scl( z[u], coeffs[s] );
-            }
+                out[o[u]] = scl( z[u], h[u] );
     } );
 }
 
@@ -192,18 +170,20 @@ __global__ void __launch_bounds__( 256 )
 
 // partial[b * S + s] = sum over this block's bins in shell s of Re(conj(G_i) X_i), in FP64.
 // A thread keeps its sum in a register while its bins stay in one shell and adds it to the
-// block's LDS sums when the shell changes: neighbouring bins share shells, and one LDS
-// atomic per bin had 64 lanes meet on a few addresses (256^3, 32 shells: 77 us, 1.8 TB/s;
-// now 38 us, 3.5 TB/s, bound by the integer work per bin: 1024-thread blocks change nothing).
+// block's LDS sums when the shell changes.  The shell changes at most bins where there are
+// many (79 % of them at 256^3 with 32 shells, 98 % at 128^3 with 100); with few, the register
+// keeps 64 lanes off a handful of addresses.  256^3 FP32 with the reduction, microseconds with
+// 1 / 8 / 32 / 100 / 1024 shells: 23.7 / 24.9 / 31.5 / 25.5 / 28.0 (24.5 / 28.6 / 39.2 / 35.2 / 104
+// with a walk over a table of shell bounds from the last bin's shell, 114 / 151 / 196 / 196 / 197
+// with an atomic and a division per bin); 128^3 with 1024: 86 -> 12.
 template <typename T>
 __global__ void __launch_bounds__( 512 ) k_shell_partials( const spec_walk w, int S, int64_t kmax2, const cpx<T> *G,
                                                            const cpx<T> *X, double *partial )
 {
     extern __shared__ double acc[];
-    int                     *thr = reinterpret_cast<int *>( acc + S );
     for ( int s = threadIdx.x; s < S; s += 512 )
         acc[s] = 0.0;
-    shell_bounds( thr, S, kmax2 );
+    __syncthreads();
     int    s   = -1;
     double sum = 0.0;
     walk_rows( w, [&]( const int64_t( &o )[4], const int( &k2 )[4], const int( & )[4] ) {
@@ -215,17 +195,17 @@ __global__ void __launch_bounds__( 512 ) k_shell_partials( const spec_walk w, in
             a[u]            = G[j];
             b[u]            = X[j];
         }
-        if ( s < 0 )
-            s = shell_of( k2[0], S, kmax2 );
 #pragma unroll
         for ( int u = 0; u < 4; ++u )
             if ( o[u] < w.total )
             {
-                if ( k2[u] < thr[s] || k2[u] >= thr[s + 1] )
+                const int t = shell_of( k2[u], S, kmax2 );
+                if ( t != s )
                 {
-                    atomicAdd( &acc[s], sum );
+                    if ( s >= 0 )
+                        atomicAdd( &acc[s], sum );
                     sum = 0.0;
-                    s   = shell_from( thr, s, k2[u] );
+                    s   = t;
                 }
                 sum += (double)a[u].x * (double)b[u].x + (double)a[u].y * (double)b[u].y;
             }
