@@ -143,12 +143,14 @@ uint32_t mulhi_magic( int64_t d )
 // fitted to 30 000 measured (schedule, cols, nt) of 31 lengths 12..2000 in all kinds, 2^22
 // and 2^25 values: the choice takes 1.03..1.05 times the best measured time there, the
 // fixed-size tiles before it 1.07..1.14.
-double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool loadb, int64_t cols, int nt,
+double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool loadb, bool pairs, int64_t cols, int nt,
                  int64_t lines )
 {
     double slots = 0, trips = 0;
+    bool   three = csize == 16 && N * csize > 16384; // a kernel of three waves per SIMD
     for ( int i = 0; i < s.n; ++i )
     {
+        three = three || ( csize == 16 && s.r[i] > 1 && !any_common_radix( s.r[i], csize ) );
         const int64_t k = ( N / s.r[i] * cols + nt - 1 ) / nt;
         if ( k > any_butterflies( s.r[i], csize ) )
             return -1;
@@ -165,15 +167,21 @@ double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool
     const double conflict = std::max( 0, ( s.r[0] & -s.r[0] ) - 2 );
     const double row      = std::max( 0.0, 1.0 - cols * csize / 128.0 );
     const double sector   = loadb && cols * csize < 32 ? 10 : 0; // below one only where nothing else fits
-    const double fill     = std::max( 0.0, 2.0 - 2.0 * (double)( ( lines + cols - 1 ) / cols ) / 512.0 );
+    const double tiles    = (double)( ( lines + cols - 1 ) / cols );
+    const double fill     = std::max( 0.0, 2.0 - 2.0 * tiles / 512.0 );
+    // Five waves and more put two on a SIMD: with three waves per SIMD a CU then holds one
+    // workgroup, not three.  2^22 values, FP64 rows of 1500 points: 320 threads 40 us (R2C) and
+    // 61 (C2C), 256 24 and 36; of 1575 41 and 62, 24 and 37; columns C2C 82, 54.  (Columns of
+    // real lines lose as much by the narrower row segments.)
+    const double crowd    = three && per_wg > 4 && tiles > 256 && ( !loadb || !pairs ) ? 20 : 0;
     if ( csize == 8 )
         return loadb ? 1 + sector + fill + 0.8 * slots + 0.8 * waves + 0.1 * octaves + 0.05 * conflict + 0.3 * inflight -
                            0.8 * first + 0.8 * row
                      : 1 + fill + 0.8 * slots + 0.8 * waves + 0.1 * octaves + 0.05 * conflict - 0.1 * first + 0.1 * lds / 65536 +
                            0.1 / 16 * ( (double)( N * cols ) / nt );
-    return loadb ? 1 + sector + fill + 0.8 * slots + 0.5 * octaves + 0.3 * conflict + 0.8 * inflight - 0.3 * first +
+    return loadb ? 1 + sector + crowd + fill + 0.8 * slots + 0.5 * octaves + 0.3 * conflict + 0.8 * inflight - 0.3 * first +
                        0.8 * lds / 65536
-                 : 1 + fill + 0.5 * slots + 0.3 * octaves + 0.05 * conflict - 0.1 * first + 0.3 * trips + 0.8 * lds / 65536;
+                 : 1 + crowd + fill + 0.5 * slots + 0.3 * octaves + 0.05 * conflict - 0.1 * first + 0.3 * trips + 0.8 * lds / 65536;
 }
 
 // Schedule and tile of a runtime-length pass; false if the length is out of range.
@@ -216,7 +224,7 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
                 for ( int nt = (int)std::max<int64_t>( 64, v0 / 64 * 64 );
                       nt <= any_max_threads( csize ) && nt <= v1 + 64; nt += 64 )
                 {
-                    const double v = any_cost( s, N, line, csize, loadb, c, nt, lines );
+                    const double v = any_cost( s, N, line, csize, loadb, kind != KIND_C2C, c, nt, lines );
                     if ( v >= 0 && ( best < 0 || v < best ) )
                     {
                         best   = v;
