@@ -31,13 +31,18 @@ constexpr int ANY_MAX_COLS    = 64; // lines per workgroup
 constexpr int any_max_threads( int csize ) { return csize == 8 ? 1024 : 512; }
 
 // Values a thread may hold in a stage (csize: bytes of a complex value), and the whole
-// butterflies of radix R that makes (one of a radix beyond it).
-constexpr int any_values( int csize ) { return csize == 8 ? 16 : 10; }
-constexpr int any_butterflies( int R, int csize )
+// butterflies of radix R that makes (one of a radix beyond it).  The FP64 kernels of lengths
+// whose table stays in memory (memtw) have radix 13 and its registers anyway and hold two
+// butterflies of radix 7: with one, lines from 1792 points with a factor 7 need five waves,
+// which leaves a CU to one workgroup (rows of 1960 points, 2^22 values: C2C 61.1 -> 40.1 us, R2C
+// 40.7 -> 26.1; 133..137 registers either way).
+constexpr int any_values( int csize, bool memtw ) { return csize == 8 ? 16 : ( memtw ? 14 : 10 ); }
+constexpr int any_butterflies( int R, int csize, bool memtw )
 {
-    const int n = any_values( csize ) / R;
+    const int n = any_values( csize, memtw ) / R;
     return n < 1 ? 1 : ( n > 4 ? 4 : n );
 }
+constexpr bool any_memtw( int64_t N, int csize ) { return N * csize > 16384; }
 // The kernels that most lengths use have the common radices and read their twiddles from an
 // LDS copy of the table.  A length with a factor 11 or 13 takes kernels that have every radix
 // (their butterflies need more registers, which the other lengths would pay for in
@@ -133,7 +138,7 @@ struct any_kernel
     template <int R, bool FIRST, bool LAST>
     __device__ static __forceinline__ void stage( const ctx &x, const any_stage s )
     {
-        constexpr int         NB    = any_butterflies( R, (int)sizeof( C ) );
+        constexpr int         NB    = any_butterflies( R, (int)sizeof( C ), MODE == ANY_MEMTW );
         const pass_params<T> &p     = x.p;
         const any_plan       &a     = x.a;
         const int             items = s.nbf * a.cols;

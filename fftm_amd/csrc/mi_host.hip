@@ -147,17 +147,18 @@ double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool
                  int64_t lines )
 {
     double slots = 0, trips = 0;
-    bool   three = csize == 16 && N * csize > 16384; // a kernel of three waves per SIMD
+    const bool memtw = any_memtw( N, csize );
+    bool       three = csize == 16 && memtw; // a kernel of three waves per SIMD
     for ( int i = 0; i < s.n; ++i )
     {
         three = three || ( csize == 16 && s.r[i] > 1 && !any_common_radix( s.r[i], csize ) );
         const int64_t k = ( N / s.r[i] * cols + nt - 1 ) / nt;
-        if ( k > any_butterflies( s.r[i], csize ) )
+        if ( k > any_butterflies( s.r[i], csize, memtw ) )
             return -1;
         slots += (double)( k * s.r[i] * nt ) / (double)( N * cols * s.n );
         trips += (double)k / s.n;
     }
-    const double lds      = (double)( line * cols * csize + ( N * csize <= 16384 ? N * csize : 0 ) );
+    const double lds      = (double)( line * cols * csize + ( memtw ? 0 : N * csize ) );
     const int    per_wg   = nt / 64, cap = csize == 8 ? 24 : 20; // wavefronts; registers allow `cap` per CU
     const int    wgs      = std::max( 1, std::min( (int)( lds_limit_wide_bytes() / lds ), cap / per_wg ) );
     const double waves    = std::max( 0.0, 1.0 - wgs * per_wg / 24.0 );
@@ -260,7 +261,7 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
     a.mg_cols = mulhi_magic( a.cols );
     a.elems   = (int32_t)( line * a.cols );
     // the LDS copy of the twiddle table up to 16 KB (32 KB cost FP64 2..6 %)
-    if ( a.nst > 1 && N * csize > 16384 )
+    if ( a.nst > 1 && any_memtw( N, csize ) )
         a.mode = ANY_MEMTW;
     return true;
 }

@@ -42,7 +42,7 @@ def _pass_us(n, kind, rows, lines, real, reps=7, calls=10):
 # 1440 = 10 8 6 3 is four stages, as every length here at most; a stage is under a third of the
 # time that the memory takes: 1.4 holds for any of them that is not short of wavefronts
 @pytest.mark.parametrize("kind", ["c2c", "r2c", "c2r"])
-@pytest.mark.parametrize("n", [1350, 1500, 1575])
+@pytest.mark.parametrize("n", [1350, 1500, 1575, 1960, 2016])
 def test_long_fp64_rows(gpu, n, kind):
     values = 1 << 22
     ref = _pass_us(1440, kind, True, values // 1440, "float64")
