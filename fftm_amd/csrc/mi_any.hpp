@@ -28,6 +28,7 @@ namespace fftm_mi
 
 constexpr int ANY_MAX_STAGES  = 5;
 constexpr int ANY_MAX_COLS    = 64; // lines per workgroup
+constexpr int ANY_STAGE_LOADS = 9;  // bins that a thread has in flight while a C2R tile is staged
 constexpr int any_max_threads( int csize ) { return csize == 8 ? 1024 : 512; }
 
 // Values a thread may hold in a stage (csize: bytes of a complex value), and the whole
@@ -375,7 +376,7 @@ struct any_kernel
         const any_plan       &a     = x.a;
         const int             lines = 2 * a.cols;
         const int             items = lines * a.nh;
-        constexpr int         U     = 9;
+        constexpr int         U     = ANY_STAGE_LOADS;
         if constexpr ( !LOADB )
         {
             // dense rows: the tile's half spectra are one contiguous piece of the array (a

@@ -202,6 +202,18 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
         any_schedules( N, csize, 16, any_schedule{}, found );
     const int64_t line = std::max<int64_t>( N, kind == KIND_C2R ? 2 * a.nh : 0 ); // LDS values per line (pair)
     const int64_t lines = kind == KIND_C2C ? ncols : ( ncols + 1 ) / 2;
+    // An array of few tiles is bound by one tile's chain of latencies: no larger ones than fill a
+    // 64-byte row or a wave where that leaves under 128 of them.  Real columns that the L2 caches
+    // hold take less: 16-byte rows on the real side (R2C of 31 columns of 1029 points FP32 11.7 ->
+    // 7.3 us, C2R of 171 of 1080 12.7 -> 9.5; larger arrays lose up to 18 % that way).  A C2R tile
+    // is staged before its first stage: rows, and FP32 columns in the caches, take a tile per CU
+    // before they take larger ones (13240 rows of 14 points 7.2 -> 5.6; FP64 columns lose up to 13 %).
+    const bool cached    = ncols * N <= 1 << 19;
+    const bool staged    = kind == KIND_C2R && ( !loadb || ( cached && csize == 8 ) );
+    int64_t    few_cols  = loadb ? ( cached && kind != KIND_C2C ? 16 : 64 ) / csize : ( 320 + N - 1 ) / N;
+    int64_t    few_tiles = staged ? 256 : 128;
+    if ( staged && !loadb )
+        few_cols = 1;
     double        best = -1;
     any_schedule  sch;
     for ( any_schedule s : found )
@@ -216,16 +228,18 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
             {
                 if ( c > 1 && line * c * csize > ( loadb ? 81920 : 45056 ) )
                     break;
-                // an array of few tiles is bound by one tile's chain of latencies: no larger
-                // ones than fill a 64-byte row or a wave where that leaves under 128 of them
-                if ( c > ( loadb ? 64 / csize : ( 320 + N - 1 ) / N ) && ( lines + c - 1 ) / c < 128 )
+                if ( c > few_cols && ( lines + c - 1 ) / c < few_tiles )
                     break;
                 // threads that hold about 5 to 16 values each
                 const int64_t v0 = N * c / 16, v1 = N * c / 5;
                 for ( int nt = (int)std::max<int64_t>( 64, v0 / 64 * 64 );
                       nt <= any_max_threads( csize ) && nt <= v1 + 64; nt += 64 )
                 {
-                    const double v = any_cost( s, N, line, csize, loadb, kind != KIND_C2C, c, nt, lines );
+                    double v = any_cost( s, N, line, csize, loadb, kind != KIND_C2C, c, nt, lines );
+                    // no second trip of staging loads in a small array (22267 rows of 14 points FP32
+                    // 7.4 -> 5.9, level beyond)
+                    if ( v >= 0 && kind == KIND_C2R && cached && line * c > ANY_STAGE_LOADS * nt )
+                        v += 0.5;
                     if ( v >= 0 && ( best < 0 || v < best ) )
                     {
                         best   = v;

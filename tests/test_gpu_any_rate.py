@@ -49,3 +49,24 @@ def test_long_fp64_rows(gpu, n, kind):
     got = _pass_us(n, kind, True, values // n, "float64")
     print(f"[rate] fp64 {kind} rows of {n}: {got:.1f} us, of 1440: {ref:.1f}", flush=True)
     assert got <= 1.4 * ref
+
+
+# arrays of at most 2^19 values lie in the L2 caches: strided lines cost address arithmetic, no
+# more than a third of such a pass
+@pytest.mark.parametrize("kind", ["r2c", "c2r"])
+@pytest.mark.parametrize("n,lines", [(1029, 31), (1029, 180), (1080, 171), (1125, 164)])
+def test_few_real_columns(gpu, n, lines, kind):
+    ref = _pass_us(n, kind, True, lines, "float32")
+    got = _pass_us(n, kind, False, lines, "float32")
+    print(f"[rate] fp32 {kind} {lines} columns of {n}: {got:.1f} us, rows: {ref:.1f}", flush=True)
+    assert got <= 1.4 * ref
+
+
+# the same bytes the other way, and one trip through LDS more
+@pytest.mark.parametrize("n,lines,rows", [(14, 13240, True), (14, 22267, True), (15, 12357, True), (14, 22267, False),
+                                          (15, 20782, False)])
+def test_short_c2r_lines(gpu, n, lines, rows):
+    ref = _pass_us(n, "r2c", rows, lines, "float32")
+    got = _pass_us(n, "c2r", rows, lines, "float32")
+    print(f"[rate] fp32 {lines} lines of {n}: c2r {got:.1f} us, r2c: {ref:.1f}", flush=True)
+    assert got <= 1.4 * ref
