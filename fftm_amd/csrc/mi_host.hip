@@ -680,7 +680,9 @@ int default_order( const pass_rt &p )
 //     -> 46.8), level with 0 and 2 within it for FP32 and 13 % slower;
 //   columns, N = 128, FP64: split exchange (6), 64 x 128 x 1024 26.2 -> 24.1, level below 32 MB;
 //   FP32 real rows, N = 64 and 256: 2 (R2C 12.6 -> 11.5, 27.0 -> 26.3; C2R 13.6 -> 12.3, 27.4
-//     -> 26.2), N = 128 R2C: 6 within the cache (27.7 -> 25.6), 5 beyond it (431 -> 403);
+//     -> 26.2); N = 128 R2C: 6 for arrays of 36..112 MB (36 MB 16.5 -> 15.1, 64 MB 24.1 -> 23.0; to
+//     32 MB 4 % slower in small arrays and level at the end, 128 MB 51.2 -> 52.6), 5 from 192 MB
+//     (224 MB 101.5 -> 99.0);
 //   FP16-stored columns: 6 where FP16 lines are read (512^3 157 -> 141, 197 -> 188, 177 ->
 //     164; shape 7 before: 192, 254, 246), 2 where they are only written or N >= 1024;
 //   hi + lo storage: 6 below N = 512, 2 from there (105 against 115); FP16-reading C2R: 2.
@@ -703,7 +705,7 @@ int default_shape( const pass_rt &p, int csize )
         if ( csize != 8 || p.loadb )
             return 0;
         if ( p.N == 128 && p.kind == KIND_R2C )
-            return beyond ? 5 : 6;
+            return bytes > (int64_t)176 << 20 ? 5 : ( bytes > 34 << 20 && bytes <= 112 << 20 ? 6 : 0 );
         return p.N == 64 || p.N == 256 ? 2 : 0;
     }
     if ( !p.loadb )
