@@ -674,8 +674,8 @@ int default_order( const pass_rt &p )
 //     with full row segments (3): 1024 x 1024 x 256 FP32 x 943 -> 534, y 496 -> 454, FP64
 //     1024 x 512 x 256 885 -> 577; arrays that the cache holds are 2-15 % better off with 2
 //     (FP32 1024 x 128 x 128 31.9 -> 29.0 against 34.0; FP64 1024 x 129 6.0 against 8.7), from
-//     2048 points on only below 32 MB (FP32 2048 columns of 2048 points 19.1 -> 17.8, 512 of them
-//     10.4 against 14.4; FP64 4096 points 27.3 -> 23.6 at 512 columns, 18.6 level at 256);
+//     2048 points on only to 16 MB (shape 2 against 3: FP32 2048 points 16 MB 12.5 and 15.4, 20 MB
+//     16.6 and 15.5, 64 MB 34.9 and 29.5; FP64 4096 points 17.4 and 18.7, 26.4 and 20.6, 52.2 and 36.7);
 //   columns, N = 256: 3 beyond the cache (256 x 1024 x 512 FP32 221 -> 193, 256^3 FP64 49.0
 //     -> 46.8), level with 0 and 2 within it for FP32 and 13 % slower;
 //   columns, N = 128, FP64: split exchange (6), 64 x 128 x 1024 26.2 -> 24.1, level below 32 MB;
@@ -710,7 +710,7 @@ int default_shape( const pass_rt &p, int csize )
     }
     if ( !p.loadb )
         return 0;
-    const bool wide = p.N >= 2048 ? bytes >= 32 << 20 : beyond;
+    const bool wide = p.N >= 2048 ? bytes > 17 << 20 : beyond;
     if ( p.N >= 512 )
         return p.N >= 1024 && wide ? 3 : 2;
     if ( p.N == 256 )

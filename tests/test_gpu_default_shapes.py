@@ -28,3 +28,12 @@ def _shape(dims, real, backward, index):
                                         ((2048, 128, 128), 0), ((3584, 128, 128), 5)])
 def test_fp32_r2c_rows_of_128(gpu, dims, shape):
     assert _shape(dims, "float32", 0, 0) == shape
+
+
+# full row segments as soon as one round of tiles does not hold the array
+@pytest.mark.parametrize("real", ["float32", "float64"])
+@pytest.mark.parametrize("n,mb,shape", [(2048, 8, 2), (2048, 16, 2), (2048, 20, 3), (2048, 64, 3), (4096, 12, 2), (4096, 16, 2),
+                                        (4096, 24, 3), (4096, 32, 3), (1024, 64, 2)])
+def test_long_columns(gpu, n, mb, shape, real):
+    columns = (mb << 20) // (n * (8 if real == "float32" else 16))
+    assert _shape((n, columns // 8, 14), real, 0, 2) == shape
