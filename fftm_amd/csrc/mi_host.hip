@@ -288,7 +288,8 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
 //   FP32 R2C rows to 288 points 1.0..3.2 (the compiled tiles hold few values per thread there
 //     and read 4-byte reals), to 480 0.96..1.2, to 1152 1.0..1.4 up to 2^23 values;
 //   FP32 C2C rows from 24 to 56 points 1.0..1.7, to 480 0.93..1.5 where the odd part is above 5
-//     or the power of two below 32, 12 points 1.3 from 2^20 values (0.9 below);
+//     or the power of two below 32; shorter ones that are one butterfly of the runtime kernel (no
+//     exchange through LDS: 12 points) 1.3 from 2^20 values (0.9 below);
 //   FP32 C2R rows of 8 times an odd number to 120 points 0.97..1.7, 2^k 7 and 2^k 9 from 112 to
 //     480 points 0.94..1.3;
 //   FP32 rows from 1000 points where radices up to 16 save a stage and the odd part is above 15:
@@ -325,8 +326,9 @@ bool runtime_faster( const pass_rt &p, int csize )
     case KIND_R2C: return N <= 288 || ( N <= 480 && within ) || ( N <= 1152 && values <= 1 << 23 );
     case KIND_C2R: return within && ( ( two == 8 && N <= 120 ) || ( two >= 16 && N <= 480 && ( odd == 7 || odd == 9 ) ) );
     default:
-        return N < 24 ? N == 12 && values >= 1 << 20
-                      : N <= 56 || ( N <= 480 && within && ( odd > 5 || two < 32 ) );
+        if ( N < 24 ) // one butterfly against two stages
+            return any_common_radix( (int)N, csize ) && values >= 1 << 20;
+        return N <= 56 || ( N <= 480 && within && ( odd > 5 || two < 32 ) );
     }
 }
 
