@@ -336,11 +336,10 @@ bool runtime_faster( const pass_rt &p, int csize )
 // plan = false: only whether it can run (every 13-smooth length in range has a plan).
 int configure_kernel( pass_rt &p, int prec, bool plan )
 {
-    if ( fixed_supported( p.N ) &&
-         !( plan && runtime_faster( p, csize_of( prec ) ) &&
-            make_any_plan( p.N, csize_of( prec ), p.loadb, p.kind, p.ncols, p.any ) ) )
+    const int cs = csize_of( prec );
+    if ( fixed_supported( p.N ) )
     {
-        p.generic = false;
+        p.generic = plan && runtime_faster( p, cs ) && make_any_plan( p.N, cs, p.loadb, p.kind, p.ncols, p.any );
         return ok();
     }
     int64_t m = p.N;
@@ -351,9 +350,7 @@ int configure_kernel( pass_rt &p, int prec, bool plan )
         return fail( FFTM_MI_NOT_SUPPORTED,
                      "fftm_mi: transform length " + std::to_string( p.N ) +
                          " has a prime factor above 13 (not supported yet)" );
-    const int cs = csize_of( prec );
-    if ( ( !fixed_supported( p.N ) && 2 * p.N * cs > 65536 ) ||
-         ( plan && !make_any_plan( p.N, cs, p.loadb, p.kind, p.ncols, p.any ) ) )
+    if ( 2 * p.N * cs > 65536 || ( plan && !make_any_plan( p.N, cs, p.loadb, p.kind, p.ncols, p.any ) ) )
         return fail( FFTM_MI_NOT_SUPPORTED,
                      "fftm_mi: transform length " + std::to_string( p.N ) + " exceeds the single-pass limit" );
     p.generic = true;
