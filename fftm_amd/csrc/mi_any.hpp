@@ -37,10 +37,10 @@ constexpr int any_max_threads( int csize ) { return csize == 8 ? 1024 : 512; }
 // butterflies of radix 7: with one, lines from 1792 points with a factor 7 need five waves,
 // which leaves a CU to one workgroup (rows of 1960 points, 2^22 values: C2C 61.1 -> 40.1 us, R2C
 // 40.7 -> 26.1; 133..137 registers either way).
-constexpr int any_values( int csize, bool memtw ) { return csize == 8 ? 16 : ( memtw ? 14 : 10 ); }
+constexpr int any_values( int csize ) { return csize == 8 ? 16 : 10; }
 constexpr int any_butterflies( int R, int csize, bool memtw )
 {
-    const int n = any_values( csize, memtw ) / R;
+    const int n = R == 7 && memtw ? 2 : any_values( csize ) / R;
     return n < 1 ? 1 : ( n > 4 ? 4 : n );
 }
 constexpr bool any_memtw( int64_t N, int csize ) { return N * csize > 16384; }

@@ -143,18 +143,21 @@ uint32_t mulhi_magic( int64_t d )
 // fitted to 30 000 measured (schedule, cols, nt) of 31 lengths 12..2000 in all kinds, 2^22
 // and 2^25 values: the choice takes 1.03..1.05 times the best measured time there, the
 // fixed-size tiles before it 1.07..1.14.
-double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool loadb, bool pairs, int64_t cols, int nt,
-                 int64_t lines )
+double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool loadb, int kind, int64_t cols, int nt,
+                 int64_t ncols )
 {
-    double slots = 0, trips = 0;
-    const bool memtw = any_memtw( N, csize );
-    bool       three = csize == 16 && memtw; // a kernel of three waves per SIMD
+    const int64_t lines = kind == KIND_C2C ? ncols : ( ncols + 1 ) / 2;
+    double        slots = 0, trips = 0;
+    const bool    memtw = any_memtw( N, csize );
+    bool          three = csize == 16 && memtw; // a kernel of three waves per SIMD
+    bool          more  = false;                // than the FP64 kernels otherwise hold
     for ( int i = 0; i < s.n; ++i )
     {
         three = three || ( csize == 16 && s.r[i] > 1 && !any_common_radix( s.r[i], csize ) );
         const int64_t k = ( N / s.r[i] * cols + nt - 1 ) / nt;
         if ( k > any_butterflies( s.r[i], csize, memtw ) )
             return -1;
+        more = more || k > any_butterflies( s.r[i], csize, false );
         slots += (double)( k * s.r[i] * nt ) / (double)( N * cols * s.n );
         trips += (double)k / s.n;
     }
@@ -172,17 +175,22 @@ double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool
     const double fill     = std::max( 0.0, 2.0 - 2.0 * tiles / 512.0 );
     // Five waves and more put two on a SIMD: with three waves per SIMD a CU then holds one
     // workgroup, not three.  2^22 values, FP64 rows of 1500 points: 320 threads 40 us (R2C) and
-    // 61 (C2C), 256 24 and 36; of 1575 41 and 62, 24 and 37; columns C2C 82, 54.  (Columns of
-    // real lines lose as much by the narrower row segments.)
-    const double crowd    = three && per_wg > 4 && tiles > 256 && ( !loadb || !pairs ) ? 20 : 0;
+    // 61 (C2C), 256 24 and 36; of 1575 41 and 62, 24 and 37; columns C2C 82, 54.  Of the strided
+    // lines only C2C of 2^21..2^23 values: with fewer the tiles do not fill the CUs, more lie beyond
+    // the memory-side cache, and real ones are pairs; there wider rows are worth as much.  More
+    // butterflies per thread only to stay at four waves.
+    const bool   part     = loadb && kind == KIND_C2C && ( ncols * N <= 1 << 21 || ncols * N > 1 << 23 );
+    const bool   wide     = per_wg > 4;
+    const double crowd    = three && wide && tiles > 256 && ( !loadb || ( kind == KIND_C2C && !part ) ) ? 20 : 0;
+    const double held     = more && ( wide || tiles <= 256 || part ) ? 20 : 0;
     if ( csize == 8 )
         return loadb ? 1 + sector + fill + 0.8 * slots + 0.8 * waves + 0.1 * octaves + 0.05 * conflict + 0.3 * inflight -
                            0.8 * first + 0.8 * row
                      : 1 + fill + 0.8 * slots + 0.8 * waves + 0.1 * octaves + 0.05 * conflict - 0.1 * first + 0.1 * lds / 65536 +
                            0.1 / 16 * ( (double)( N * cols ) / nt );
-    return loadb ? 1 + sector + crowd + fill + 0.8 * slots + 0.5 * octaves + 0.3 * conflict + 0.8 * inflight - 0.3 * first +
+    return loadb ? 1 + sector + crowd + held + fill + 0.8 * slots + 0.5 * octaves + 0.3 * conflict + 0.8 * inflight - 0.3 * first +
                        0.8 * lds / 65536
-                 : 1 + crowd + fill + 0.5 * slots + 0.3 * octaves + 0.05 * conflict - 0.1 * first + 0.3 * trips + 0.8 * lds / 65536;
+                 : 1 + crowd + held + fill + 0.5 * slots + 0.3 * octaves + 0.05 * conflict - 0.1 * first + 0.3 * trips + 0.8 * lds / 65536;
 }
 
 // Schedule and tile of a runtime-length pass; false if the length is out of range.
@@ -203,17 +211,16 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
     const int64_t line = std::max<int64_t>( N, kind == KIND_C2R ? 2 * a.nh : 0 ); // LDS values per line (pair)
     const int64_t lines = kind == KIND_C2C ? ncols : ( ncols + 1 ) / 2;
     // An array of few tiles is bound by one tile's chain of latencies: no larger ones than fill a
-    // 64-byte row or a wave where that leaves under 128 of them.  Real columns that the L2 caches
-    // hold take less: 16-byte rows on the real side (R2C of 31 columns of 1029 points FP32 11.7 ->
-    // 7.3 us, C2R of 171 of 1080 12.7 -> 9.5; larger arrays lose up to 18 % that way).  A C2R tile
-    // is staged before its first stage: rows, and FP32 columns in the caches, take a tile per CU
-    // before they take larger ones (13240 rows of 14 points 7.2 -> 5.6; FP64 columns lose up to 13 %).
-    const bool cached    = ncols * N <= 1 << 19;
-    const bool staged    = kind == KIND_C2R && ( !loadb || ( cached && csize == 8 ) );
-    int64_t    few_cols  = loadb ? ( cached && kind != KIND_C2C ? 16 : 64 ) / csize : ( 320 + N - 1 ) / N;
-    int64_t    few_tiles = staged ? 256 : 128;
-    if ( staged && !loadb )
-        few_cols = 1;
+    // 64-byte row or a wave where that leaves under 128 of them.  FP32 real columns of at most 2^18
+    // values, which an L2 cache holds, and up to 2^20 where there are no more pairs than CUs, take
+    // less: 16-byte rows on the real side (R2C of 31 columns of 1029 points 11.7 -> 7.3 us, C2R of 171
+    // of 1080 12.7 -> 8.4; more pairs of 2^19 values lose up to 36 %, FP64 ones up to 13 %).  A C2R tile
+    // is staged before its first stage: such columns take a tile per CU and rows 320 tiles before
+    // they take larger ones (13240 rows of 14 points 7.2 -> 5.6).
+    const int64_t values    = ncols * N;
+    const bool    few       = kind != KIND_C2C && csize == 8 && ( values <= 1 << 18 || ( lines <= 256 && values <= 1 << 20 ) );
+    const int64_t few_cols  = loadb ? ( few ? 16 : 64 ) / csize : ( kind == KIND_C2R ? 1 : ( 320 + N - 1 ) / N );
+    const int64_t few_tiles = kind != KIND_C2R || ( loadb && !few ) ? 128 : ( loadb ? 256 : 320 );
     double        best = -1;
     any_schedule  sch;
     for ( any_schedule s : found )
@@ -235,10 +242,11 @@ bool make_any_plan( int64_t N, int csize, bool loadb, int kind, int64_t ncols, a
                 for ( int nt = (int)std::max<int64_t>( 64, v0 / 64 * 64 );
                       nt <= any_max_threads( csize ) && nt <= v1 + 64; nt += 64 )
                 {
-                    double v = any_cost( s, N, line, csize, loadb, kind != KIND_C2C, c, nt, lines );
-                    // no second trip of staging loads in a small array (22267 rows of 14 points FP32
-                    // 7.4 -> 5.9, level beyond)
-                    if ( v >= 0 && kind == KIND_C2R && cached && line * c > ANY_STAGE_LOADS * nt )
+                    double v = any_cost( s, N, line, csize, loadb, kind, c, nt, ncols );
+                    // no second trip of staging loads in a small array (22267 columns of 14 points
+                    // FP32 7.5 -> 5.6, level beyond; FP64 columns are better off with wider rows)
+                    if ( v >= 0 && kind == KIND_C2R && values <= 1 << 19 && ( !loadb || csize == 8 ) &&
+                         line * c > ANY_STAGE_LOADS * nt )
                         v += 0.5;
                     if ( v >= 0 && ( best < 0 || v < best ) )
                     {
