@@ -2,8 +2,8 @@
 // radices up to 16, the same Stockham stages, address maps and real-axis handling as the
 // compile-time pass kernel (mi_pass.hpp).
 //
-// The host picks a schedule with as few stages as the radices allow (250 = 5 5 10,
-// 1080 = 9 10 12), a tile of `cols` lines and a workgroup in which every thread holds whole
+// The host picks a schedule with as few stages as the radices allow (FP32: 250 = 10 5 5,
+// 1080 = 15 12 6), a tile of `cols` lines and a workgroup in which every thread holds whole
 // butterflies of at most any_values() values per stage (any_plan).  A stage is then: read
 // the thread's butterflies (stage 0 from HBM, the others from LDS), twiddle, DFT in
 // registers, write back to the one LDS tile (the last stage of a C2C or C2R pass straight to
@@ -14,11 +14,15 @@
 // otherwise, for the loads as for the stores.
 //
 // Bound by memory latency and, next to it, by the integer and twiddle work per value.
-// Batches of 2^23 complex values, FP32 rows / columns: N = 250 25.5 / 28.1 us (5.3 / 4.8
-// TB/s), N = 1080 26.2 / 33.0 us; FP64 250: 44.9 / 48.4 us (6.0 / 5.6 TB/s).  Its
+// Batches of 2^23 complex values, FP32 rows / columns: N = 250 24.9 / 27.7 us (5.4 / 4.8
+// TB/s), N = 1080 27.2 / 31.8 us; FP64 250: 41.9 / 48.6 us (6.4 / 5.5 TB/s).  Its
 // predecessor, one radix per thread and ping-pong LDS buffers with every line transformed
-// column-fastest, took 76 / 75, 60 / 68 and 102 / 101 us.  With the tile chosen by
-// any_cost, the 175 x 250 x 330 FP32 pair went from 180 (tiles of a fixed size) to 171 us.
+// column-fastest, took 79 / 76, 59 / 69 and 104 / 101 us.  With the tile chosen by
+// any_cost, the 175 x 250 x 330 FP32 pair went from 180 (tiles of a fixed size) to 172 us.
+//
+// Registers: FP32 common radices 79..80, every radix 82..87, table in memory 93..96; FP64 93..97
+// and 133..137.  The FP32 C2R kernels and the strided R2C one of the common radices keep 2..4 of
+// theirs in scratch memory (12 bytes per lane) to stay at six waves per SIMD.
 #pragma once
 
 #include "mi_pass.hpp"

@@ -140,9 +140,10 @@ uint32_t mulhi_magic( int64_t d )
 // The terms: lanes idle in some stage (1: none), wavefronts per CU short of 24, octaves off
 // 256 threads, bank conflicts of stage 0's writes (stride r0), bytes in flight per CU short
 // of 128 KB, loads per thread in stage 0, trips per stage, LDS, short rows.  The weights were
-// fitted to 30 000 measured (schedule, cols, nt) of 31 lengths 12..2000 in all kinds, 2^22
-// and 2^25 values: the choice takes 1.03..1.05 times the best measured time there, the
-// fixed-size tiles before it 1.07..1.14.
+// fitted to measured tiles of 31 lengths 12..2000.  With every (first radix, cols, nt) of 4134
+// arrays timed (92 lengths 5..4004, all kinds and both mappings, 2^13..2^22.3 values), the choice
+// takes 1.07 times the best of them: FP64 1.03..1.09 by kind, mapping and size, FP32 rows
+// 1.03..1.14, columns 1.06..1.15.
 double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool loadb, int kind, int64_t cols, int nt,
                  int64_t ncols )
 {
@@ -692,7 +693,9 @@ int default_order( const pass_rt &p )
 //     (224 MB 101.5 -> 99.0);
 //   FP16-stored columns: 6 where FP16 lines are read (512^3 157 -> 141, 197 -> 188, 177 ->
 //     164; shape 7 before: 192, 254, 246), 2 where they are only written or N >= 1024;
-//   hi + lo storage: 6 below N = 512, 2 from there (105 against 115); FP16-reading C2R: 2.
+//   hi + lo storage: 6 below N = 512, 2 from there (105 against 115); FP16-reading C2R to N = 512:
+//     2 (whole pairs, 128^3 48.6 -> 48.3, 128 x 128 x 512 82.7 -> 80.5, 256^3 134.7 -> 133.2, 512^3
+//     1023 -> 1015, hi + lo 256^3 166.6 -> 164.0; level at 256 x 512 x 256).
 int default_shape( const pass_rt &p, int csize )
 {
     if ( p.plane || p.generic || !pow2_length( p.N ) || p.N < 64 )

@@ -400,6 +400,8 @@ struct plane_rx_geom
 //   32 points, 1024 planes: 5.1 / 5.8 -> 5.1 / 5.3, 6.8 / 7.0 -> 6.4 / 6.6; 4096: 10.5 / 11.3 ->
 //   11.8 / 12.0.
 // The 64-point planes of a 64^4 pencil (4096) take 149 us a pair without, 155 with.
+// Registers at 128 points FP64: 154..158 without, 109 (forward) and 128 (inverse) with; the wide
+// inverse keeps 4 values of them in scratch memory (20 bytes per lane).
 inline bool plane_rx_wide( int n, int csize, int64_t nplanes )
 {
     return n >= 128 ? csize == 16 || nplanes <= 256 : nplanes <= 1024;

@@ -3,7 +3,7 @@
 //
 // Problems of a few thousand points are bound by their launches: a 12 x 10 x 8 FP64 pair
 // took six kernels of 3 to 5.5 us, each nearly all latency, 28 us in all; two of these take
-// 16.5, 16^3 23 instead of 27.  They are bound by one wave's chain of latencies (about 1300
+// 16.4, 16^3 23 instead of 27.  They are bound by one wave's chain of latencies (about 1300
 // instructions for 4^3), so the loops divide by multiplying and no stage's indices are formed
 // ahead of its turn.  Here the array stays in LDS
 // from the first load to the last store.  Every radix stage of every axis reads one LDS
@@ -11,6 +11,9 @@
 // one writes HBM.  Real rows are transformed in pairs as in the pass kernel; the separation
 // of a pair is folded into the reads of the first complex axis, the Hermitian extension of
 // the backward transform into the reads of the real axis.
+//
+// Every radix to 16 of both kinds of axis is in one kernel: 72 / 124 registers FP32 forward /
+// inverse, 128 / 194 FP64 (two waves per SIMD), and 108..392 scalar values kept in vector lanes.
 #pragma once
 
 #include "mi_any.hpp"

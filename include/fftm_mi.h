@@ -66,8 +66,9 @@ extern "C" {
  * input-sized complex buffer.  With this flag the input is used as scratch
  * (hipFFT's documented out-of-place C2R behaviour) and the work size is 0. */
 #define FFTM_MI_FLAG_OVERWRITE_INPUT 1
-/* ffts handles: keep the real axis and its partner axis in separate passes instead of
- * one plane pass (used to measure the fusion; results are the same within rounding). */
+/* ffts handles: a pass per axis.  No plane pass for the real axis and its partner axis, no
+ * pass over the planes of the two inner axes, no volume pass for a whole small transform
+ * (used to measure the fusions; results are the same within rounding). */
 #define FFTM_MI_FLAG_NO_PLANE_FUSION 2
 
 /*
