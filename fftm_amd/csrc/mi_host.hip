@@ -141,7 +141,7 @@ uint32_t mulhi_magic( int64_t d )
 // 256 threads, bank conflicts of stage 0's writes (stride r0), bytes in flight per CU short
 // of 128 KB, loads per thread in stage 0, trips per stage, LDS, short rows.  The weights were
 // fitted to measured tiles of 31 lengths 12..2000.  With every (first radix, cols, nt) of 4134
-// arrays timed (92 lengths 5..4004, all kinds and both mappings, 2^13..2^22.3 values), the choice
+// arrays timed (75 lengths 5..4004, all kinds and both mappings, 2^13..2^22.3 values), the choice
 // takes 1.07 times the best of them: FP64 1.03..1.09 by kind, mapping and size, FP32 rows
 // 1.03..1.14, columns 1.06..1.15.
 double any_cost( const any_schedule &s, int64_t N, int64_t line, int csize, bool loadb, int kind, int64_t cols, int nt,
@@ -1369,9 +1369,14 @@ void fuse_tiles( const ffts_layout &L, int32_t layout, int prec, std::vector<pas
          !make_tile( L, csize_of( prec ), d - 2, d - 2, p.vol ) )
         return;
     // 12 waves per CU in all: enough to hide latency, and no more threads per plane than that
-    // takes (3000 planes of 40 x 30 FP32 75 -> 72 us with 64 threads instead of 256)
-    vol_geom &v = p.vol;
-    v.nt        = (int32_t)std::min<int64_t>( v.nt, std::max<int64_t>( 1, ( 3072 + planes / 2 ) / planes ) * 64 );
+    // takes (3000 planes of 40 x 30 FP32 75 -> 72 us with 64 threads instead of 256); and no more than
+    // let a CU hold all the planes that fall to it, at the inverse kernel's four (FP32) or two
+    // (FP64) waves per SIMD: a fifth wave takes a second one of a SIMD (572 planes of 44 x 39 FP64,
+    // pair 84.3 us with five waves, 70.5 with four)
+    vol_geom     &v    = p.vol;
+    const int64_t deep = ( csize_of( prec ) == 8 ? 4 : 2 ) / ( ( planes + 255 ) / 256 );
+    const int64_t want = std::max<int64_t>( 1, std::min( ( 3072 + planes / 2 ) / planes, 4 * std::max<int64_t>( 1, deep ) ) );
+    v.nt        = (int32_t)std::min<int64_t>( v.nt, want * 64 );
     v.blocks    = (int32_t)planes;
     v.bd0       = (int32_t)L.n[d - 3];
     for ( int i = 0; i < d - 2; ++i )
