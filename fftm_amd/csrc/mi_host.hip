@@ -1337,20 +1337,21 @@ void fuse_volume( const ffts_layout &L, int prec, std::vector<pass_rt> &fwd, std
 
 // Whether a launch of `planes` volume-pass workgroups, one per plane of the real axis (nb) and
 // its neighbour (na), beats the two passes it replaces.  Transform pairs, time of the passes
-// over the tile's, 80 shapes of 2^13..2^23 points drawn over both layouts and precisions:
-//   planes of at most 60 KB LDS: 1.02..1.34 (36 x 30 x 40 x 24 FP64 67 -> 63 us, FP32 53 -> 44,
-//     64 x 16 x 64 x 32 FP32 63 -> 55, 512 x 48 x 28 FP64 52 -> 40), but FP64 arrays of many
-//     planes or beyond 1.5 million points, where the arithmetic per value counts, 0.94..0.99,
-//     and FP32 ones beyond 6 million (2000 x 60 x 60 106 -> 108, 72^4 362 -> 492);
-//   larger planes (one or two workgroups per CU): 1.03..1.29 from 72 planes to one per CU
-//     (128 x 64 x 100 FP64 53 -> 41), 0.77..0.97 with fewer or more, and 0.96 above 136 KB; 0.90
-//     where the real rows are powers of two (128 x 64 x 128 FP64 45.5 -> 50).
+// over the tile's, 2421 arrays of 2^13..2^22.6 points that took a tile, both layouts and precisions:
+//   planes of at most 60 KB LDS: 1.05..1.17 on average by layout, precision and which lengths are
+//     powers of two; FP32 from 2^20 points 1.15..1.18 up to 4.2 million, 1.00 from there to 4.7
+//     million (5 arrays, 0.90..1.16), 0.92 beyond (11 arrays, 0.85..0.99: all lose);
+//   larger planes (one or two workgroups per CU): 1.05..1.17 from 72 planes to one per CU.
+// 47 of the 2410 within these lines lose more than 2 %, the worst 15 %.  The other sides, from 80
+// shapes drawn the same way: FP64 arrays of many planes or beyond 1.5 million points 0.94..0.99;
+// larger planes 0.77..0.97 with fewer planes or more, 0.96 above 136 KB, and 0.90 where the real
+// rows are powers of two (128 x 64 x 128 FP64 45.5 -> 50 us).
 bool tile_faster( int64_t planes, int64_t na, int64_t nb, int csize )
 {
     const int64_t lds = 2 * csize * std::max( na * ( nb / 2 + 1 ), ( na + 1 ) / 2 * nb );
     if ( lds > 60 * 1024 )
         return lds <= 136 * 1024 && planes >= 72 && planes <= 256 && !pow2_length( nb );
-    return planes >= 24 && ( csize == 8 ? planes * na * nb <= 6 << 20 : planes <= 2304 && planes * na * nb <= 3 << 19 );
+    return planes >= 24 && ( csize == 8 ? planes * na * nb <= 9 << 19 : planes <= 2304 && planes * na * nb <= 3 << 19 );
 }
 
 // Replace the real-axis pass and its neighbour's by one volume pass per plane where no plane

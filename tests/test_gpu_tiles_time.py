@@ -1,6 +1,6 @@
 """A pass per plane of the two inner axes where it is the faster way: against a pass per axis of the
 same library, at plane counts between one and three per CU (the workgroups of a CU have to be
-resident together)."""
+resident together) and at the size from which arithmetic decides."""
 
 import ctypes
 import math
@@ -56,3 +56,11 @@ def test_planes_share_a_cu(gpu, real, dims):
         L.fftm_mi_ffts_destroy(h)
     print(f"[tiles] {real} {dims}: per plane {us[0]:.1f} us, per axis {us[_lib.FLAG_NO_PLANE_FUSION]:.1f}", flush=True)
     assert us[0] <= 1.1 * us[_lib.FLAG_NO_PLANE_FUSION]
+
+
+@pytest.mark.parametrize("dims,passes", [((64, 64, 16, 64), 3), ((50, 48, 60, 39), 4), ((42, 40, 56, 64), 4)])
+def test_large_fp32_arrays_take_a_pass_per_axis(gpu, dims, passes):
+    from fftm_amd import _lib
+    h = _handle(_lib.LAYOUT_4D_SLAB, dims, "float32", 0)
+    assert _passes(h) == passes
+    _lib.lib().fftm_mi_ffts_destroy(h)
